@@ -59,18 +59,25 @@ template <> struct Mfma32<f16_t> {
 constexpr int kChunk32Rows = 32;   // query rows per wave
 
 // LDS swizzle of a staged block: chunk c (16 B) of token t (0..15) sits at
-// slot c ^ swz(t) of the token's 256-byte row, swz(4a + b) = 4b + a.  The
-// q . k reads (one chunk, 16 tokens per 16 lanes) meet 16 distinct slots
-// mod 16, and so do the V transpose reads (chunks c0 .. c0 + 3, c0 a
-// multiple of 4, of four consecutive tokens 4a .. 4a + 3 per 32 lanes): each
-// group of accesses covers every 16-byte bank group once.
-__device__ __forceinline__ int swz(int t) { return ((t & 3) << 2) | (t >> 2); }
-// P . V with the weights split into 16-bit hi and lo parts (1) or rounded
-// once to 16 bits (0: the default — a query chunk is bound by the matrix
-// cores, and the single rounding stays far inside the tolerance)
+// slot c ^ swz(t) of the token's row.  The q . k reads (one chunk, 16 tokens
+// per 16 lanes) meet 16 distinct slots mod 16, and so do the V transpose reads
+// (chunks c0 .. c0 + 3, c0 a multiple of 4, of four consecutive tokens
+// 4a .. 4a + 3 per 32 lanes): each group of accesses covers every 16-byte bank
+// group once.  Rows of 256 bytes or more (D = 128, 256): swz(4a + b) = 4b + a.
+// D = 64, two tokens per 256 bytes: the eight tokens of one parity take eight
+// different XORs, t and t + 2 differing in bit 2, swz(4a + 2b + p) = 4b + a.
+template <int D>
+__device__ __forceinline__ int swz(int t) {
+  return D == 64 ? ((t & 2) << 1) | (t >> 2) : ((t & 3) << 2) | (t >> 2);
+}
+// P . V with the weights split into 16-bit hi and lo parts or, at D = 128,
+// rounded once to 16 bits (a query chunk is bound by the matrix cores, and the
+// single rounding stays far inside the tolerance; HELM_CHUNK32_HILO=1 builds
+// the split there too)
 #ifndef HELM_CHUNK32_HILO
 #define HELM_CHUNK32_HILO 0
 #endif
+constexpr bool chunk32_hilo(int D) { return D != 128 || HELM_CHUNK32_HILO; }
 constexpr float kLog2E = 1.4426950408889634f;   // log2(e)
 constexpr float kLn2 = 0.6931471805599453f;     // ln(2)
 
@@ -84,25 +91,30 @@ __device__ __forceinline__ void buf_load16_lds(__amdgpu_buffer_rsrc_t r, void* l
 
 // NW waves per workgroup (4: two workgroups per CU; 8: one, which halves the
 // stage loads per query row), 32 query rows each.
-template <typename T, class Src, int FEAT, int NW>
-__global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, Src src) {
+template <typename T, class Src, int FEAT, int NW, int D>
+__device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src& src) {
   static_assert(NW == 4 || NW == 8, "waves per workgroup");
   constexpr int SB = kChunkStage;   // 16-token blocks per stage
+  constexpr bool kHiLo = chunk32_hilo(D);
+  constexpr int NK = D / 16;        // 16-dim steps of q . k
+  constexpr int NE = D / 32;        // 32-dim groups of P . V
+  constexpr int CPR = D / 8;        // 16-byte chunks per token row
   using Ops = MfmaOps<T>;
   using M32 = Mfma32<T>;
-  constexpr int kRow = 256;                // bytes per token row (128 dims x 2 B)
-  constexpr int kBlk = kBlockTok * kRow;   // 4 KiB per 16-token block of K (or V)
+  constexpr int kRow = 2 * D;              // bytes per token row
+  constexpr int kBlk = kBlockTok * kRow;   // bytes per 16-token block of K (or V)
   constexpr bool kMask = (FEAT & kFeatMask) != 0;
   constexpr bool kCap = (FEAT & kFeatCap) != 0;
   constexpr bool kCausal = (FEAT & kFeatCausal) != 0;
   // 16-byte-per-lane loads (1 KiB each) a wave issues per stage: a stage is
-  // SB blocks of K and of V, 4 loads each, shared out over the NW waves in
-  // order (wave w takes loads w * kLoads ..), all in one block per wave
-  constexpr int kLoads = 8 * SB / NW;
+  // SB blocks of K and of V, kBlkLoads loads each, shared out over the NW
+  // waves in order (wave w takes loads w * kLoads ..), all in one block per wave
+  constexpr int kBlkLoads = kBlk / 1024;
+  constexpr int kLoads = 2 * kBlkLoads * SB / NW;
   // two stage buffers as two objects, so that the compiler sees that the
   // loads filling one never touch the reads of the other:
   // [K, V][block of the stage][16-byte chunk], chunk c of token t at slot
-  // t * 16 + (c ^ swz(t)) (see swz)
+  // t * CPR + (c ^ swz(t)) (see swz)
   typedef mf_u32x4 StageBuf[2][SB][kBlk / 16];
   __shared__ StageBuf lds0, lds1;
 
@@ -130,7 +142,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
   auto out_elem = [&](int g, int t, int e) -> uint16_t* {
     const RowCoord c = row_coord(rbase + 8 * g + 4 * hh + t, G);
     return reinterpret_cast<uint16_t*>(p.out) +
-           ((int64_t)(b * p.Hq + hk * G + c.g) * S + c.s) * 128 + 32 * e + jr;
+           ((int64_t)(b * p.Hq + hk * G + c.g) * S + c.s) * D + 32 * e + jr;
   };
 
   const int np = src.n_pages(b);
@@ -151,7 +163,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
         for (int t = 0; t < 4; ++t)
           if (8 * g + 4 * hh + t < nrows)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) *out_elem(g, t, e) = 0;
+            for (int e = 0; e < NE; ++e) *out_elem(g, t, e) = 0;
     }
     return;
   }
@@ -168,12 +180,12 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
   const int s_vis = s_row + coff;                      // row jr's last visible token
   const int s_last = (rbase + nrows - 1) / G + coff;   // the wave's last visible token
   const int s_first = rbase / G + coff;                // and its first row's
-  mf_u32x4 qop[8];
+  mf_u32x4 qop[NK];
   {
     const char* qp = reinterpret_cast<const char*>(p.q) +
                      ((int64_t)(b * p.Hq + hk * G + rc.g) * S + s_row) * kRow;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NK; ++i) {
       const uint4 v = *reinterpret_cast<const uint4*>(qp + 16 * (2 * i + hh));
       qop[i] = row_ok ? mf_u32x4{v.x, v.y, v.z, v.w} : mf_u32x4{0u, 0u, 0u, 0u};
     }
@@ -190,20 +202,17 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
   auto sexp = [](float v) { return __builtin_amdgcn_exp2f(v); };
 
   float m = -INFINITY;   // running max of row jr (same in both halves)
-#if HELM_CHUNK32_HILO
-  float lsum = 0.f;      // this lane's share of the row's weight sum
-#else
-  // the rows' weight sums on the matrix cores: P times a column of ones, so
-  // the sum takes exactly the 16-bit weights that P . V takes; register
+  float lsum = 0.f;      // hi + lo: this lane's share of the row's weight sum
+  // else the rows' weight sums on the matrix cores: P times a column of ones,
+  // so the sum takes exactly the 16-bit weights that P . V takes; register
   // 4g + t holds row 8g + 4hh + t (the same value in every lane of a half)
   mf_f32x16 osum;
 #pragma unroll
   for (int r = 0; r < 16; ++r) osum[r] = 0.f;
   const mf_u32x4 ones = Ops::ones8();
-#endif
-  mf_f32x16 o[4];
+  mf_f32x16 o[NE];
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
+  for (int e = 0; e < NE; ++e)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[e][r] = 0.f;
 
@@ -225,7 +234,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
     int ntok;
     const char *kb, *vb;
   };
-  const int own_blk = (wave * kLoads) >> 3;
+  const int own_blk = (wave * kLoads) / (2 * kBlkLoads);
   // (a stage never straddles two record windows: window w starts at block
   // 64 w bpp of the split, a multiple of the stage's SB = 4 blocks, so the
   // window is entered at a stage's first block; blocks past the split's end
@@ -261,21 +270,21 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
   };
 
   // this wave's loads of a stage straight from memory into LDS (no VGPRs):
-  // load i = wave * kLoads + k covers K (bit 2 of i clear) or V of the
-  // wave's block, slots 64u .. 64u + 63 with u = i % 4, lane l slot 64u + l,
-  // which holds chunk (l & 15) ^ swz(t) of token t = 4u + (l >> 4) (the
-  // swizzle), so each lane fetches that chunk; loads past the block's tokens
-  // write zeros
+  // load i = wave * kLoads + k covers K (the block's first kBlkLoads) or V of
+  // the wave's block, slots 64u .. 64u + 63 with u = i % kBlkLoads, lane l slot
+  // 64u + l of token t = (64u + l) / CPR, which holds chunk (l % CPR) ^ swz(t)
+  // (the swizzle), so each lane fetches that chunk; loads past the block's
+  // tokens write zeros
   auto dma_stage = [&](const OwnBlock& ob, StageBuf& dst) {
     const auto rk = make_rsrc(ob.kb, ob.ntok * kRow);
     const auto rv = make_rsrc(ob.vb, ob.ntok * kRow);
 #pragma unroll
     for (int k = 0; k < kLoads; ++k) {
       const int i = wave * kLoads + k;
-      const int u = i & 3;
-      const int t = 4 * u + (lane >> 4);
-      const int off = t * kRow + 16 * ((lane & 15) ^ swz(t));
-      if ((i >> 2) & 1)
+      const int u = i % kBlkLoads;
+      const int t = (64 / CPR) * u + lane / CPR;
+      const int off = t * kRow + 16 * ((lane % CPR) ^ swz<D>(t));
+      if ((i / kBlkLoads) & 1)
         buf_load16_lds(rv, &dst[1][own_blk][64 * u], off);
       else
         buf_load16_lds(rk, &dst[0][own_blk][64 * u], off);
@@ -292,7 +301,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
   auto vaddr = [&](const StageBuf& cur, int blk, int z, int e) -> const char* {
     const int vtok = 8 * hh + 4 * z + (nl >> 2);
     const int chunk = 4 * e + 2 * (jr >> 4) + ((nl & 3) >> 1);
-    return reinterpret_cast<const char*>(&cur[1][blk][vtok * 16 + (chunk ^ swz(vtok))]) +
+    return reinterpret_cast<const char*>(&cur[1][blk][vtok * CPR + (chunk ^ swz<D>(vtok))]) +
            8 * (nl & 1);
   };
 
@@ -362,14 +371,14 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
         // then the eight MFMAs back to back), registers allowing: with a mask
         // operand its prefetched values take them, and the compiler's order
         // stays
-        mf_u32x4 ka[8];
+        mf_u32x4 ka[NK];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          ka[i] = cur[0][bp + kblk][ktok * 16 + ((2 * i + hh) ^ swz(ktok))];
-        if constexpr (!kMask)
+        for (int i = 0; i < NK; ++i)
+          ka[i] = cur[0][bp + kblk][ktok * CPR + ((2 * i + hh) ^ swz<D>(ktok))];
+        if constexpr (!kMask && D == 128)
           __builtin_amdgcn_sched_barrier(0);   // (keeps the reads ahead of the MFMAs)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) sc = M32::mma(ka[i], qop[i], sc);
+        for (int i = 0; i < NK; ++i) sc = M32::mma(ka[i], qop[i], sc);
         return sc;
       };
       // steps that add exactly nothing for any row of the wave are skipped
@@ -422,14 +431,14 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
           // refresh the row max (both halves of the row agree)
           const float mn = fmaxf(m, fmaxf(bm, __shfl_xor(bm, 32, 64)));
           const float a = sexp(m - ((mn == -INFINITY) ? 0.f : mn));
-#if HELM_CHUNK32_HILO
-          lsum *= a;
-#else
+          if constexpr (kHiLo) {
+            lsum *= a;
+          } else {
 #pragma unroll
-          for (int g = 0; g < 4; ++g)
+            for (int g = 0; g < 4; ++g)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) osum[4 * g + t] *= __shfl(a, 8 * g + 4 * hh + t, 64);
-#endif
+              for (int t = 0; t < 4; ++t) osum[4 * g + t] *= __shfl(a, 8 * g + 4 * hh + t, 64);
+          }
           m = mn;
           // O register 4g + t is row 8g + 4hh + t: that row's factor
 #pragma unroll
@@ -438,7 +447,7 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
             for (int t = 0; t < 4; ++t) {
               const float ar = __shfl(a, 8 * g + 4 * hh + t, 64);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) o[e][4 * g + t] *= ar;
+              for (int e = 0; e < NE; ++e) o[e][4 * g + t] *= ar;
             }
         }
         const float base = (m == -INFINITY) ? 0.f : m;
@@ -446,34 +455,33 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           const float w0 = sexp(x[2 * q] - base), w1 = sexp(x[2 * q + 1] - base);
-#if HELM_CHUNK32_HILO
-          lsum += w0 + w1;
-          Ops::split2(w0, w1, hw[q], lw[q]);
-#else
-          hw[q] = Ops::pk(w0, w1);
-          lw[q] = 0u;
-#endif
+          if constexpr (kHiLo) {
+            lsum += w0 + w1;
+            Ops::split2(w0, w1, hw[q], lw[q]);
+          } else {
+            hw[q] = Ops::pk(w0, w1);
+            lw[q] = 0u;
+          }
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const mf_u32x4 phi = mf_u32x4{hw[4 * u], hw[4 * u + 1], hw[4 * u + 2], hw[4 * u + 3]};
           const mf_u32x4 plo = mf_u32x4{lw[4 * u], lw[4 * u + 1], lw[4 * u + 2], lw[4 * u + 3]};
-          mf_u32x4 vop[4];
+          mf_u32x4 vop[NE];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
+          for (int e = 0; e < NE; ++e) {
             const uint2 a0 = ld_tr16(vaddr(cur, bp + u, 0, e));
             const uint2 a1 = ld_tr16(vaddr(cur, bp + u, 1, e));
             vop[e] = mf_u32x4{a0.x, a0.y, a1.x, a1.y};
           }
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = M32::mma(phi, vop[e], o[e]);
-#if HELM_CHUNK32_HILO
+          for (int e = 0; e < NE; ++e) o[e] = M32::mma(phi, vop[e], o[e]);
+          if constexpr (kHiLo) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) o[e] = M32::mma(plo, vop[e], o[e]);
-#else
-          (void)plo;
-          osum = M32::mma(phi, ones, osum);
-#endif
+            for (int e = 0; e < NE; ++e) o[e] = M32::mma(plo, vop[e], o[e]);
+          } else {
+            osum = M32::mma(phi, ones, osum);
+          }
         }
       };
       {
@@ -514,17 +522,18 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
   }
 
   if (!wave_rows) return;
-#if HELM_CHUNK32_HILO
-  const float lrow = lsum + __shfl_xor(lsum, 32, 64);     // row jr's sum
-#else
-  // row jr's sum: held by the half hh = (jr >> 2) & 1, register 4 (jr >> 3) + (jr & 3)
-  float lself = 0.f;
+  float lrow;     // row jr's sum
+  if constexpr (kHiLo) {
+    lrow = lsum + __shfl_xor(lsum, 32, 64);
+  } else {
+    // held by the half hh = (jr >> 2) & 1, register 4 (jr >> 3) + (jr & 3)
+    float lself = 0.f;
 #pragma unroll
-  for (int r = 0; r < 16; ++r)
-    if (r == 4 * (jr >> 3) + (jr & 3)) lself = osum[r];
-  const float lother = __shfl_xor(lself, 32, 64);
-  const float lrow = (((jr >> 2) & 1) == hh) ? lself : lother;
-#endif
+    for (int r = 0; r < 16; ++r)
+      if (r == 4 * (jr >> 3) + (jr & 3)) lself = osum[r];
+    const float lother = __shfl_xor(lself, 32, 64);
+    lrow = (((jr >> 2) & 1) == hh) ? lself : lother;
+  }
   if (p.direct_out) {
     // the call's only split: normalized rows straight to the output
     // (HELM's final out / max(sum, 1e-12), kv_cache.py:554-555)
@@ -533,19 +542,15 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int i = 8 * g + 4 * hh + t;
-#if HELM_CHUNK32_HILO
-        const float inv = 1.f / fmaxf(__shfl(lrow, i, 64), 1e-12f);
-#else
-        const float inv = 1.f / fmaxf(osum[4 * g + t], 1e-12f);
-#endif
+        const float inv = 1.f / fmaxf(kHiLo ? __shfl(lrow, i, 64) : osum[4 * g + t], 1e-12f);
         if (i < nrows)
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
+          for (int e = 0; e < NE; ++e)
             *out_elem(g, t, e) = static_cast<uint16_t>(Ops::pk(o[e][4 * g + t] * inv, 0.f));
       }
     return;
   }
-  // partials (m, l, o[128]) of the wave's rows in their 16-row tiles
+  // partials (m, l, o[D]) of the wave's rows in their 16-row tiles
   auto part_row = [&](int i) -> int64_t {
     return ((int64_t)(tile0 + (i >> 4)) * p.max_splits + split) * p.rows_per_tile + (i & 15);
   };
@@ -558,11 +563,28 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
     for (int t = 0; t < 4; ++t) {
       const int i = 8 * g + 4 * hh + t;
       if (i < nrows) {
-        float* dst = &p.ws_o[part_row(i) * 128 + jr];
+        float* dst = &p.ws_o[part_row(i) * D + jr];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) dst[32 * e] = o[e][4 * g + t];
+        for (int e = 0; e < NE; ++e) dst[32 * e] = o[e][4 * g + t];
       }
     }
+}
+
+template <typename T, class Src, int FEAT, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, Src src) {
+  chunk32_mfma_body<T, Src, FEAT, NW, 128>(p, src);
+}
+// D = 64: 32 KiB of LDS and under 128 registers.  D = 256: the 128 KiB of its
+// two stage buffers leave one workgroup per CU, and its 32 x 256 O tile and
+// 32 x 256 query operand take 192 registers before any score: one wave per
+// SIMD, which may use all 512.  Against the vector-ALU kernel, which read K
+// and V once per four rows: f16 D = 64, 777 tokens over 2,777 (14 / 2 heads),
+// 436 -> 33 us; bf16 D = 256, 512 over 4,700 soft-capped under a window mask
+// (16 / 8 heads), 3,033 -> 203 us.
+template <typename T, class Src, int FEAT, int NW, int D>
+__global__ __launch_bounds__(NW * 64, D == 256 ? 1 : 2) void chunk32_mfma_dim_kernel(AttnParams p,
+                                                                                     Src src) {
+  chunk32_mfma_body<T, Src, FEAT, NW, D>(p, src);
 }
 
 }  // namespace helm

@@ -6,23 +6,10 @@
 #include "attn_kernel.h"
 #include "attn_mfma.h"
 #include "attn_chunk32.h"
-
-#include <hip/hip_ext.h>
+#include "attn_launch.h"
 
 namespace helm {
 namespace {
-
-// A launch timed by helm_profile_split_kernels goes through
-// hipExtLaunchKernelGGL with the spec's start / stop events, which then carry
-// the kernel's own start and end; every other launch is a plain launch.
-#define HELM_ATTN_LAUNCH(KERNEL, GRID, BLOCK, ...)                                       \
-  do {                                                                                   \
-    if (s.ev_start)                                                                      \
-      hipExtLaunchKernelGGL(KERNEL, GRID, BLOCK, 0, st, s.ev_start, s.ev_stop, 0,        \
-                            __VA_ARGS__);                                                \
-    else                                                                                 \
-      hipLaunchKernelGGL(KERNEL, GRID, BLOCK, 0, st, __VA_ARGS__);                       \
-  } while (0)
 
 template <typename TKV, typename TQ, int EPL, int GM, bool DOT2>
 hipError_t launch_one(const LaunchSpec& s, hipStream_t st) {

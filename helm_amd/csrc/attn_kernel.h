@@ -762,19 +762,20 @@ __device__ __forceinline__ void split_epilogue(Smem<NW, GM, DMAX>& sm, const Att
     fused_merge_tail<TQ, NW, GM, DMAX>(sm, p, tid, tile, total, nrows, r0, b, hk);
 }
 
-// The same end of a split for the matrix-core kernel (D = 128, GM rows): the
+// The same end of a split for the matrix-core kernel (GM rows of D dims): the
 // waves' row states are merged and each row's partial goes out as 16-byte
 // stores, with the column arithmetic fixed at compile time.
-template <typename TQ, int NW, int GM>
-__device__ __forceinline__ void split_epilogue_d128(Smem<NW, GM, 128>& sm, const AttnParams& p,
+template <typename TQ, int NW, int GM, int D>
+__device__ __forceinline__ void split_epilogue_mfma(Smem<NW, GM, D>& sm, const AttnParams& p,
                                                     int tid, int tile, int split, int total,
                                                     int nrows, int r0, int b, int hk) {
   constexpr int NT = 64 * NW;
+  constexpr int DC = D / 4;   // float4 columns of a row
   const int64_t part = ((int64_t)tile * p.max_splits + split) * p.rows_per_tile;
   const auto pr = partials_rsrc(p);
-  for (int idx = tid; idx < nrows * 32; idx += NT) {
-    const int g = idx >> 5;
-    const int d0 = (idx & 31) * 4;
+  for (int idx = tid; idx < nrows * DC; idx += NT) {
+    const int g = idx / DC;
+    const int d0 = (idx % DC) * 4;
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, sm.m[w][g]);
@@ -789,10 +790,10 @@ __device__ __forceinline__ void split_epilogue_d128(Smem<NW, GM, 128>& sm, const
       O.x += a * v.x; O.y += a * v.y; O.z += a * v.z; O.w += a * v.w;
     }
     if (p.fused) {
-      st_coherent16(pr, (part + g) * 128 + d0, O);
+      st_coherent16(pr, (part + g) * D + d0, O);
       if (d0 == 0) st_agent_ml(&p.ws_ml[(part + g) * 2], M, L);
     } else {
-      *reinterpret_cast<float4*>(&p.ws_o[(part + g) * 128 + d0]) = O;
+      *reinterpret_cast<float4*>(&p.ws_o[(part + g) * D + d0]) = O;
       if (d0 == 0) *reinterpret_cast<float2*>(&p.ws_ml[(part + g) * 2]) = make_float2(M, L);
     }
   }
@@ -806,14 +807,14 @@ __device__ __forceinline__ void split_epilogue_d128(Smem<NW, GM, 128>& sm, const
     __syncthreads();
     if (!sm.last) return;
     constexpr int QB = ElemBytes<TQ>::v;
-    const int items = nrows * 32;               // (row, float4 column chunk)
+    const int items = nrows * DC;               // (row, float4 column chunk)
     const int nsub = items >= NT ? 1 : NT / items;
     const int sub = tid / items;
     const int it = tid - sub * items;
     const int64_t part0 = (int64_t)tile * p.max_splits * p.rows_per_tile;
     for (int i = it; i < items && sub < nsub; i += NT) {
-      const int g = i >> 5;
-      const int d0 = (i & 31) * 4;
+      const int g = i / DC;
+      const int d0 = (i % DC) * 4;
       float M = -INFINITY, L = 0.f;
       float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
       constexpr int kB = 16;  // one trip for up to 16 * nsub splits
@@ -826,7 +827,7 @@ __device__ __forceinline__ void split_epilogue_d128(Smem<NW, GM, 128>& sm, const
           if (sp < total) {
             const int64_t pi = part0 + (int64_t)sp * p.rows_per_tile + g;
             ml[k] = ld_agent_ml(reinterpret_cast<const float2*>(p.ws_ml) + pi);
-            v[k] = ld_coherent16(pr, pi * 128 + d0);
+            v[k] = ld_coherent16(pr, pi * D + d0);
           } else {
             ml[k] = make_float2(-INFINITY, 0.f);
             v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -857,7 +858,7 @@ __device__ __forceinline__ void split_epilogue_d128(Smem<NW, GM, 128>& sm, const
         const RowCoord rc = row_coord(rr, p.G);
         const int h = hk * p.G + rc.g, sq = rc.s;
         char* orow =
-            reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + sq) * 128 * QB;
+            reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + sq) * D * QB;
         store_elem<TQ>(orow + (d0 + 0) * QB, acc.x * inv);
         store_elem<TQ>(orow + (d0 + 1) * QB, acc.y * inv);
         store_elem<TQ>(orow + (d0 + 2) * QB, acc.z * inv);
@@ -885,12 +886,12 @@ __device__ __forceinline__ void split_epilogue_d128(Smem<NW, GM, 128>& sm, const
         o.w = fmaf(wgt, t.w, o.w);
       }
       const float inv = 1.f / fmaxf(Lx, 1e-12f);
-      const int g = i >> 5;
-      const int d0 = (i & 31) * 4;
+      const int g = i / DC;
+      const int d0 = (i % DC) * 4;
       const int rr = r0 + g;
       const RowCoord rc = row_coord(rr, p.G);
       const int h = hk * p.G + rc.g, sq = rc.s;
-      char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + sq) * 128 * QB;
+      char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + sq) * D * QB;
       store_elem<TQ>(orow + (d0 + 0) * QB, o.x * inv);
       store_elem<TQ>(orow + (d0 + 1) * QB, o.y * inv);
       store_elem<TQ>(orow + (d0 + 2) * QB, o.z * inv);
@@ -1033,14 +1034,16 @@ __global__ __launch_bounds__(kThreads) void merge_splits_kernel(AttnParams p) {
   }
 }
 
-// merge_splits_kernel for D = 128 with one column group, the arithmetic fixed
-// at compile time: thread (sub, c) = (tid / 32, tid % 32) owns float4 column
-// chunk c and splits sub, sub + 8, ...; the 8 subs meet in LDS.  A short,
-// division-free kernel: it runs once per call with a cold instruction cache.
-template <typename TQ>
-__global__ __launch_bounds__(kThreads) void merge_splits_d128_kernel(AttnParams p) {
+// merge_splits_kernel for the matrix-core head dims (64, 128, 256) with one column group, the
+// arithmetic fixed at compile time: thread (sub, c) = (tid / (D / 4), tid %
+// (D / 4)) owns float4 column chunk c and splits sub, sub + kSub, ...; the
+// kSub subs meet in LDS (D = 128: 8 of them).  A short, division-free kernel:
+// it runs once per call with a cold instruction cache.
+template <typename TQ, int D>
+__device__ __forceinline__ void merge_splits_body(const AttnParams& p) {
   constexpr int QB = ElemBytes<TQ>::v;
-  constexpr int kSub = kThreads / 32;
+  constexpr int DC = D / 4;
+  constexpr int kSub = kThreads / DC;
   __shared__ float4 red[kThreads];
   __shared__ float2 redml[kThreads];
   const int tile = blockIdx.x;
@@ -1055,8 +1058,8 @@ __global__ __launch_bounds__(kThreads) void merge_splits_d128_kernel(AttnParams 
   const int rr = qt * RS + row;
   if (rr >= p.G * p.S) return;
   const int total = p.counts[tile];
-  const int sub = tid >> 5;
-  const int c = tid & 31;
+  const int sub = tid / DC;
+  const int c = tid % DC;
   const int64_t base_part = (int64_t)tile * p.max_splits * RS + row;
   float M = -INFINITY, L = 0.f;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1073,7 +1076,7 @@ __global__ __launch_bounds__(kThreads) void merge_splits_d128_kernel(AttnParams 
       if (sp < bound) {
         const int64_t pi = base_part + (int64_t)sp * RS;
         ml[k] = *reinterpret_cast<const float2*>(p.ws_ml + pi * 2);
-        v[k] = *reinterpret_cast<const float4*>(p.ws_o + pi * 128 + c * 4);
+        v[k] = *reinterpret_cast<const float4*>(p.ws_o + pi * D + c * 4);
       } else {
         ml[k] = make_float2(-INFINITY, 0.f);
         v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1106,17 +1109,17 @@ __global__ __launch_bounds__(kThreads) void merge_splits_d128_kernel(AttnParams 
   red[tid] = acc;
   redml[tid] = make_float2(M, L);
   __syncthreads();
-  if (tid < 32) {
+  if (tid < DC) {
     float Mx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < kSub; ++j) Mx = fmaxf(Mx, redml[tid + 32 * j].x);
+    for (int j = 0; j < kSub; ++j) Mx = fmaxf(Mx, redml[tid + DC * j].x);
     const float base = (Mx == -INFINITY) ? 0.f : Mx;
     float Lx = 0.f;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int j = 0; j < kSub; ++j) {
-      const float2 ml = redml[tid + 32 * j];
-      const float4 t = red[tid + 32 * j];
+      const float2 ml = redml[tid + DC * j];
+      const float4 t = red[tid + DC * j];
       const float wgt = fexp(ml.x - base);
       Lx = fmaf(wgt, ml.y, Lx);
       o.x = fmaf(wgt, t.x, o.x);
@@ -1127,7 +1130,7 @@ __global__ __launch_bounds__(kThreads) void merge_splits_d128_kernel(AttnParams 
     const float inv = 1.f / fmaxf(Lx, 1e-12f);
     const RowCoord rc = row_coord(rr, p.G);
     const int h = hk * p.G + rc.g, sq = rc.s;
-    char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + sq) * 128 * QB;
+    char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + sq) * D * QB;
     store_elem<TQ>(orow + (tid * 4 + 0) * QB, o.x * inv);
     store_elem<TQ>(orow + (tid * 4 + 1) * QB, o.y * inv);
     store_elem<TQ>(orow + (tid * 4 + 2) * QB, o.z * inv);
@@ -1135,23 +1138,33 @@ __global__ __launch_bounds__(kThreads) void merge_splits_d128_kernel(AttnParams 
   }
 }
 
+template <typename TQ>
+__global__ __launch_bounds__(kThreads) void merge_splits_d128_kernel(AttnParams p) {
+  merge_splits_body<TQ, 128>(p);
+}
+template <typename TQ, int D>
+__global__ __launch_bounds__(kThreads) void merge_splits_dim_kernel(AttnParams p) {
+  merge_splits_body<TQ, D>(p);
+}
+
 // The merge for calls with many query rows and few splits (query chunks):
-// thread (r, c) = (tid / 32, tid % 32) of workgroup (tile, y) owns row
-// 8 y + r of the tile and its float4 column chunk c, and walks the splits
+// thread (r, c) = (tid / DC, tid % DC), DC = D / 4, of workgroup (tile, y)
+// owns row (256 / DC) y + r of the tile and its float4 column chunk c, and walks the splits
 // itself (no reduction across threads), eight partials in flight at a time
 // (the first eight issued before the split count arrives, bounded by the
-// workspace's split capacity).  Same arithmetic as merge_splits_d128_kernel
+// workspace's split capacity).  Same arithmetic as merge_splits_body
 // per split, in split order.
-template <typename TQ>
-__global__ __launch_bounds__(kThreads) void merge_rows_d128_kernel(AttnParams p) {
+template <typename TQ, int D>
+__device__ __forceinline__ void merge_rows_body(const AttnParams& p) {
   constexpr int QB = ElemBytes<TQ>::v;
+  constexpr int DC = D / 4;
   const int tile = blockIdx.x;
   // every split of the tile has finished claiming blocks
   if (blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) reset_claims(p, tile);
   const int tid = threadIdx.x;
   const int RS = p.rows_per_tile;
-  const int row = blockIdx.y * (kThreads / 32) + (tid >> 5);
-  const int c = tid & 31;
+  const int row = blockIdx.y * (kThreads / DC) + tid / DC;
+  const int c = tid % DC;
   const int qt = tile % p.n_qtiles;
   const int hk = (tile / p.n_qtiles) % p.Hkv;
   const int b = tile / (p.n_qtiles * p.Hkv);
@@ -1172,7 +1185,7 @@ __global__ __launch_bounds__(kThreads) void merge_rows_d128_kernel(AttnParams p)
       if (sp < bound) {
         const int64_t pi = base_part + (int64_t)sp * RS;
         ml[k] = *reinterpret_cast<const float2*>(p.ws_ml + pi * 2);
-        v[k] = *reinterpret_cast<const float4*>(p.ws_o + pi * 128 + c * 4);
+        v[k] = *reinterpret_cast<const float4*>(p.ws_o + pi * D + c * 4);
       } else {
         ml[k] = make_float2(-INFINITY, 0.f);
         v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1205,11 +1218,20 @@ __global__ __launch_bounds__(kThreads) void merge_rows_d128_kernel(AttnParams p)
   const float inv = 1.f / fmaxf(L, 1e-12f);
   const RowCoord rc = row_coord(rr, p.G);
   const int h = hk * p.G + rc.g;
-  char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + rc.s) * 128 * QB;
+  char* orow = reinterpret_cast<char*>(p.out) + ((int64_t)(b * p.Hq + h) * p.S + rc.s) * D * QB;
   store_elem<TQ>(orow + (4 * c + 0) * QB, acc.x * inv);
   store_elem<TQ>(orow + (4 * c + 1) * QB, acc.y * inv);
   store_elem<TQ>(orow + (4 * c + 2) * QB, acc.z * inv);
   store_elem<TQ>(orow + (4 * c + 3) * QB, acc.w * inv);
+}
+
+template <typename TQ>
+__global__ __launch_bounds__(kThreads) void merge_rows_d128_kernel(AttnParams p) {
+  merge_rows_body<TQ, 128>(p);
+}
+template <typename TQ, int D>
+__global__ __launch_bounds__(kThreads) void merge_rows_dim_kernel(AttnParams p) {
+  merge_rows_body<TQ, D>(p);
 }
 
 template <typename TKV, typename TQ, int EPL, int GM, bool DOT2, class Src>
@@ -1593,5 +1615,10 @@ struct LaunchSpec {
 hipError_t launch_attn_f16(const LaunchSpec& s, hipStream_t st);
 hipError_t launch_attn_bf16(const LaunchSpec& s, hipStream_t st);
 hipError_t launch_attn_f32(const LaunchSpec& s, hipStream_t st);
+// The matrix-core kernels at head dims 64 and 256 (attn_dim.h).
+hipError_t launch_attn_f16_d64(const LaunchSpec& s, hipStream_t st);
+hipError_t launch_attn_f16_d256(const LaunchSpec& s, hipStream_t st);
+hipError_t launch_attn_bf16_d64(const LaunchSpec& s, hipStream_t st);
+hipError_t launch_attn_bf16_d256(const LaunchSpec& s, hipStream_t st);
 
 }  // namespace helm

@@ -1,5 +1,5 @@
 // Split-K paged decode attention on the matrix cores (gfx950 MFMA), for
-// 16-bit K/V pages with head_dim 128 — the hot configuration of HELM's
+// 16-bit K/V pages with head_dim 64, 128 or 256 — the hot configurations of HELM's
 // perform_streaming_attention (helm/runtime/kv_cache.py:468-555 masked
 // online-softmax loop, :562-568 Path 1, :584-662 Path 3) and of the batched
 // decode of _decode_batched (helm/runtime/kv_offload.py:152-174).
@@ -28,6 +28,11 @@
 //     (hi + lo) . v.  Lane (q4, n) loads V rows 4j + q4 at dims 8n..8n+7: a
 //     wave load is 1 KiB contiguous.  Products are exact and accumulate in
 //     fp32.
+// (Written for D = 128; D = 64 halves the K chunks and the dims a lane holds
+// of a V row to four, D = 256 doubles both, the V row's halves apart: VRow.
+// Against the vector-ALU kernel that served them before: f16 D = 64, four
+// sequences of 3k-16k tokens, 45.6 -> 17.6 us; bf16 D = 256, 8,000 tokens
+// soft-capped under a window mask, 37.9 -> 19.2 us.)
 // No data moves between lanes in the loop; the split's per-wave states meet in
 // LDS; the shared split epilogue (attn_kernel.h) merges the waves and then
 // the splits.
@@ -51,7 +56,8 @@ constexpr float kMfmaSlack = 8.f;
 #ifndef HELM_MFMA_NBUF
 #define HELM_MFMA_NBUF 2
 #endif
-constexpr int kMfmaBufs = HELM_MFMA_NBUF;
+// D = 64's blocks are 4 KiB of K/V: twice as many are in flight per wave.
+constexpr int mfma_bufs(int D) { return D == 64 ? 4 : HELM_MFMA_NBUF; }
 
 // kFeatMask16: the mask is 16-bit (bf16 / fp16); only the decode kernel
 // reads it at that width (the chunk kernels read the element type at run time)
@@ -61,6 +67,17 @@ typedef __bf16 mf_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 mf_f16x8 __attribute__((ext_vector_type(8)));
 typedef float mf_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t mf_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t mf_u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t mf_u32x8 __attribute__((ext_vector_type(8)));
+
+// One lane's share of a V row in the decode kernel, D / 16 dims in D / 32
+// words: lane n of a row's 16 holds dims 4n .. 4n + 3 (D = 64), 8n .. 8n + 7
+// (128) or those of both halves of the row (256: 8n .. and 128 + 8n ..), so
+// every load instruction covers whole rows contiguously.
+template <int D> struct VRow;
+template <> struct VRow<64> { typedef mf_u32x2 type; };
+template <> struct VRow<128> { typedef mf_u32x4 type; };
+template <> struct VRow<256> { typedef mf_u32x8 type; };
 
 template <typename T> struct MfmaOps;
 
@@ -118,6 +135,22 @@ template <> struct MfmaOps<f16_t> {
 __device__ __forceinline__ mf_u32x4 buf_load16_nt(__amdgpu_buffer_rsrc_t r, int off) {
   const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 2);
   return mf_u32x4{v[0], v[1], v[2], v[3]};
+}
+
+// A lane's share of a V row (VRow) at byte offset row of the resource.
+template <int D>
+__device__ __forceinline__ typename VRow<D>::type buf_load_vrow_nt(__amdgpu_buffer_rsrc_t r,
+                                                                   int row, int n) {
+  if constexpr (D == 64) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, row + 8 * n, 0, 2);
+    return mf_u32x2{v[0], v[1]};
+  } else if constexpr (D == 128) {
+    return buf_load16_nt(r, row + 16 * n);
+  } else {
+    const mf_u32x4 a = buf_load16_nt(r, row + 16 * n);
+    const mf_u32x4 b = buf_load16_nt(r, row + 256 + 16 * n);
+    return mf_u32x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  }
 }
 
 // LDS transpose read of 16-bit elements (ds_read_b64_tr_b16): within each
@@ -236,11 +269,11 @@ __device__ __forceinline__ PageMeta lane_page_meta(const DescSrc&, const DescLan
 // HELM token cursor of its first token.  Updates the row max m, this lane's
 // share of the row sum, and O (rows 4 q4 + r, dims 8n + e).
 // q . k of the lane's row n for tokens 4r + q4 of a block (K operand k).
-template <class Ops>
-__device__ __forceinline__ mf_f32x4 mfma_qk(const mf_u32x4 (&k)[4], const mf_u32x4 (&qop)[4]) {
+template <class Ops, int NK>
+__device__ __forceinline__ mf_f32x4 mfma_qk(const mf_u32x4 (&k)[NK], const mf_u32x4 (&qop)[NK]) {
   mf_f32x4 sc = mf_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sc = Ops::mma(k[i], qop[i], sc);
+  for (int i = 0; i < NK; ++i) sc = Ops::mma(k[i], qop[i], sc);
   return sc;
 }
 
@@ -270,8 +303,9 @@ __device__ __forceinline__ void mfma_logits(mf_f32x4 sc, const float (&mk)[4], i
 // The lazy online-softmax reference update for a block max bm: when bm
 // exceeds the row max by more than the slack anywhere in the wave, the row
 // max is refreshed and l and the O rows rescaled.
+template <int NO>
 __device__ __forceinline__ void mfma_refresh_max(float bm, float& m, float& lsum,
-                                                 mf_f32x4 (&o)[8], int q4) {
+                                                 mf_f32x4 (&o)[NO], int q4) {
   if (__builtin_amdgcn_ballot_w64(bm > m + kMfmaSlack)) {
     // refresh the row max (uniform across the row's four lanes)
     float rm = fmaxf(bm, __shfl_xor(bm, 16, 64));
@@ -285,16 +319,16 @@ __device__ __forceinline__ void mfma_refresh_max(float bm, float& m, float& lsum
     for (int r = 0; r < 4; ++r) {
       const float ar = __shfl(a, 4 * q4 + r, 64);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e][r] *= ar;
+      for (int e = 0; e < NO; ++e) o[e][r] *= ar;
     }
   }
 }
 
 // Weights exp(x - m) of the four tokens into l and, as hi + lo 16-bit parts,
-// P . V into O (V operand v: tokens q4 + 4j at dims 8n .. 8n + 7).
-template <class Ops>
-__device__ __forceinline__ void mfma_pv(const float (&x)[4], const mf_u32x4 (&v)[4], float m,
-                                        float& lsum, mf_f32x4 (&o)[8]) {
+// P . V into O (V operand v: tokens q4 + 4j at the lane's dims of the row).
+template <class Ops, class V, int NO>
+__device__ __forceinline__ void mfma_pv(const float (&x)[4], const V (&v)[4], float m,
+                                        float& lsum, mf_f32x4 (&o)[NO]) {
   const float base = (m == -INFINITY) ? 0.f : m;
   float wt[4];
 #pragma unroll
@@ -307,7 +341,7 @@ __device__ __forceinline__ void mfma_pv(const float (&x)[4], const mf_u32x4 (&v)
   Ops::split2(wt[2], wt[3], h23, l23);
   const mf_u32x4 pop = mf_u32x4{h01, h23, l01, l23};
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < NO / 2; ++w) {
     const uint32_t a01 = pack_lo(v[0][w], v[1][w]);
     const uint32_t a23 = pack_lo(v[2][w], v[3][w]);
     const uint32_t b01 = pack_hi(v[0][w], v[1][w]);
@@ -318,11 +352,11 @@ __device__ __forceinline__ void mfma_pv(const float (&x)[4], const mf_u32x4 (&v)
 }
 
 // One 16-token block of the recurrence: q . k, logits, max refresh, P . V.
-template <class Ops, bool kMask, bool kCap, bool kCausal>
-__device__ __forceinline__ void mfma_block_step(const mf_u32x4 (&k)[4], const mf_u32x4 (&v)[4],
+template <class Ops, bool kMask, bool kCap, bool kCausal, class V, int NK, int NO>
+__device__ __forceinline__ void mfma_block_step(const mf_u32x4 (&k)[NK], const V (&v)[4],
                                                 const float (&mk)[4], int ntok, int tok0,
-                                                const mf_u32x4 (&qop)[4], float& m, float& lsum,
-                                                mf_f32x4 (&o)[8], float scale, float cap,
+                                                const mf_u32x4 (&qop)[NK], float& m, float& lsum,
+                                                mf_f32x4 (&o)[NO], float scale, float cap,
                                                 float inv_cap, int s_vis, int q4) {
   float x[4];
   mfma_logits<kMask, kCap, kCausal>(mfma_qk<Ops>(k, qop), mk, ntok, tok0, scale, cap, inv_cap,
@@ -335,17 +369,22 @@ template <class Src> struct LanesOf;
 template <> struct LanesOf<PoolSrc> { using type = PoolLanes; };
 template <> struct LanesOf<DescSrc> { using type = DescLanes; };
 
-template <typename T, class Src, int FEAT, int NW>
-__global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src src) {
+// The decode kernel of head dim D (64, 128 or 256); the entry points below
+// launch it.
+template <typename T, class Src, int FEAT, int NW, int D>
+__device__ __forceinline__ void decode_mfma_body(const AttnParams& p, const Src& src) {
   using Ops = MfmaOps<T>;
+  using V = typename VRow<D>::type;
   constexpr int NT = 64 * NW;
-  constexpr int kRow = 256;  // bytes per token row (128 dims x 2 B)
+  constexpr int kRow = 2 * D;     // bytes per token row
+  constexpr int NK = D / 32;      // K (and Q) operand chunks of a lane
+  constexpr int NO = D / 16;      // O column groups (MFMAs of P . V per block)
   constexpr bool kMask = (FEAT & kFeatMask) != 0;
   constexpr bool kCap = (FEAT & kFeatCap) != 0;
   constexpr bool kCausal = (FEAT & kFeatCausal) != 0;
   constexpr bool kMask16 = (FEAT & kFeatMask16) != 0;
 
-  __shared__ Smem<NW, kMfmaRows, 128> sm;
+  __shared__ Smem<NW, kMfmaRows, D> sm;
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -387,7 +426,7 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
       lane_pages(src, b, p.lo + split_local * p.pps, lane);
   // a split of more than 64 pages: the records of its pages 64 .. 127
   typename LanesOf<Src>::type lanes_hi{};
-  if (p.pps > 64 && !p.dyn) lanes_hi = lane_pages(src, b, p.lo + split_local * p.pps + 64, lane);
+  if (p.pps > 64 && !(D == 128 && p.dyn)) lanes_hi = lane_pages(src, b, p.lo + split_local * p.pps + 64, lane);
   // ---- query operand: row n of the tile at dim chunks 4i + q4 ---------------
   const bool row_ok = n < nrows;
   const int rr = r0 + (row_ok ? n : 0);
@@ -396,13 +435,13 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
   const int s_row = rc.s;
   // causal: query position s sees tokens 0 .. s + causal - 1
   const int s_vis = s_row + (kCausal ? p.causal - 1 : 0);
-  mf_u32x4 qop[4];
+  mf_u32x4 qop[NK];
   {
     const int h = hk * G + g_row;
     const char* qp = reinterpret_cast<const char*>(p.q) +
                      ((int64_t)(b * p.Hq + h) * S + s_row) * kRow;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NK; ++i) {
       const uint4 v = *reinterpret_cast<const uint4*>(qp + 16 * (4 * i + q4));
       qop[i] = row_ok ? mf_u32x4{v.x, v.y, v.z, v.w} : mf_u32x4{0u, 0u, 0u, 0u};
     }
@@ -420,11 +459,11 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
   const bool active = total > 0 && split_local < nsplit_launch;
   if (!active) {
     if (total == 0 && p.fused && split_local == 0) {
-      for (int idx = tid; idx < nrows * 128; idx += NT) {
-        const int zr = r0 + idx / 128;
+      for (int idx = tid; idx < nrows * D; idx += NT) {
+        const int zr = r0 + idx / D;
         const RowCoord rc = row_coord(zr, G);
         const int h = hk * G + rc.g, s = rc.s;
-        const int64_t o_off = ((int64_t)(b * p.Hq + h) * S + s) * 128 + idx % 128;
+        const int64_t o_off = ((int64_t)(b * p.Hq + h) * S + s) * D + idx % D;
         store_elem<T>(reinterpret_cast<char*>(p.out) + o_off * 2, 0.f);
       }
     }
@@ -434,7 +473,7 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
   const int split = p.split_base + split_local;
   const int pg0 = lo + split_local * p.pps;
   const int npg = min(pg0 + p.pps, hi) - pg0;  // 1..kMfmaMaxPps
-  if constexpr (std::is_same<Src, DescSrc>::value) {
+  if constexpr (D == 128 && std::is_same<Src, DescSrc>::value) {
     // a call that carries the sequences' new tokens: each workgroup whose
     // split holds the sequence's last page writes its head's token into that
     // page's last used slot (16 lanes K, 16 lanes V, 16 bytes each), and the
@@ -465,20 +504,19 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
 
   float m = -INFINITY;  // running max of row n (same in the 4 lanes of the row)
   float lsum = 0.f;     // this lane's share of row n's weight sum
-  mf_f32x4 o[8];
+  mf_f32x4 o[NO];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int e = 0; e < NO; ++e) o[e] = mf_f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int bpp = p.bpp;
   const int nblk = npg * bpp;
   // lane offsets inside a block: K token tau(n) at chunk q4 (+64 B per i),
-  // V token q4 at dims 8n (+1 KiB per j)
+  // V token q4 (+4 rows per j)
   const int voff_k = (4 * (n & 3) + (n >> 2)) * kRow + 16 * q4;
-  const int voff_v = q4 * kRow + 16 * n;
 
   struct Blk {
-    mf_u32x4 k[4];
-    mf_u32x4 v[4];
+    mf_u32x4 k[NK];
+    V v[4];
     // mask elements as loaded, at their width (a 16-bit mask kept as 16-bit
     // values: zero-extending them would be an instruction on each loaded
     // register, placed where the next step's loads must have completed)
@@ -500,9 +538,9 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
     const auto rk = make_rsrc(pv.k + tok_in * kRow, ntok * kRow);
     const auto rv = make_rsrc(pv.v + tok_in * kRow, ntok * kRow);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) B.k[i] = buf_load16_nt(rk, voff_k + 64 * i);
+    for (int i = 0; i < NK; ++i) B.k[i] = buf_load16_nt(rk, voff_k + 64 * i);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) B.v[j] = buf_load16_nt(rv, voff_v + 1024 * j);
+    for (int j = 0; j < 4; ++j) B.v[j] = buf_load_vrow_nt<D>(rv, (q4 + 4 * j) * kRow, n);
     if constexpr (kMask) {
       // token 4r + q4 of the block for row n; clamped inside the block's
       // tokens (a block past its page's tokens reads the row's first key:
@@ -535,7 +573,7 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
   // ahead (scalar load) and the K / V of the block one ahead, then computes
   // the current block: each of the three latencies hides behind one step.
   // Claims only grow, so a wave is done at its first block past the tile.
-  if (p.dyn) {
+  if (D == 128 && p.dyn) {
     const int Wt = nsplit_launch * NW;
     const int np_t = hi - lo;
     const int nblk_t = np_t * bpp;
@@ -616,9 +654,9 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
       const auto rk = make_rsrc(pv.k, ntok * kRow);
       const auto rv = make_rsrc(pv.v, ntok * kRow);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) B.k[i] = buf_load16_nt(rk, voff_k + 64 * i);
+      for (int i = 0; i < NK; ++i) B.k[i] = buf_load16_nt(rk, voff_k + 64 * i);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) B.v[j] = buf_load16_nt(rv, voff_v + 1024 * j);
+      for (int j = 0; j < 4; ++j) B.v[j] = buf_load_vrow_nt<D>(rv, (q4 + 4 * j) * kRow, n);
       if constexpr (kMask) {
         const int mbase = ntok > 0 ? B.tok0 : 0;
         const int last = max(ntok - 1, 0);
@@ -670,7 +708,7 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
   // ---- main loop: a ring of kMfmaBufs register buffers, kMfmaBufs - 1
   // blocks' loads in flight while one block is computed ----------------------
   {
-    constexpr int NB = kMfmaBufs;
+    constexpr int NB = mfma_bufs(D);
     // this wave's blocks: wave, wave + NW, ...
     const int nmine = nblk > wave ? (nblk - wave + NW - 1) / NW : 0;
     Blk buf[NB];
@@ -707,14 +745,26 @@ __global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src 
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    float* dst = &sm.o[wave][4 * q4 + r][8 * n];
-    *reinterpret_cast<float4*>(dst) = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
-    *reinterpret_cast<float4*>(dst + 4) = make_float4(o[4][r], o[5][r], o[6][r], o[7][r]);
+    // the lane's dims: D = 64 4n .. 4n + 3, else 8n .. 8n + 7 of each 128
+    float* dst = &sm.o[wave][4 * q4 + r][(D == 64 ? 4 : 8) * n];
+#pragma unroll
+    for (int e = 0; e < NO; e += 4)
+      *reinterpret_cast<float4*>(dst + (e >> 3) * 128 + (e & 7)) =
+          make_float4(o[e][r], o[e + 1][r], o[e + 2][r], o[e + 3][r]);
   }
   __syncthreads();
   if (stp && tid == 0) stp[1] = stamp_now();
-  split_epilogue_d128<T, NW, kMfmaRows>(sm, p, tid, tile, split, total, nrows, r0, b, hk);
+  split_epilogue_mfma<T, NW, kMfmaRows, D>(sm, p, tid, tile, split, total, nrows, r0, b, hk);
   if (stp && tid == 0) stp[2] = stamp_now();
+}
+
+template <typename T, class Src, int FEAT, int NW>
+__global__ __launch_bounds__(64 * NW) void decode_mfma_kernel(AttnParams p, Src src) {
+  decode_mfma_body<T, Src, FEAT, NW, 128>(p, src);
+}
+template <typename T, class Src, int FEAT, int D>
+__global__ __launch_bounds__(256) void decode_mfma_dim_kernel(AttnParams p, Src src) {
+  decode_mfma_body<T, Src, FEAT, 4, D>(p, src);
 }
 
 // ---- query chunks: K/V blocks staged through LDS ----------------------------

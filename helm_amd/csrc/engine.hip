@@ -131,9 +131,9 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // ---- kernel choice and split planning -----------------------------------
 // Three kernels, chosen per call:
-//   mfma    — matrix-core kernel (attn_mfma.h): 16-bit q == KV type, D = 128,
-//             16-byte aligned operands; up to 16 query rows per tile;
-//   fast    — vector-ALU dot2 kernel: same types, G <= 8 rows per tile;
+//   mfma    — matrix-core kernel (attn_mfma.h): 16-bit q == KV type, D = 64,
+//             128 or 256, 16-byte aligned operands; up to 16 query rows per tile;
+//   fast    — vector-ALU dot2 kernel: same types, D = 128, G <= 8 rows per tile;
 //   generic — any D <= 256, fp32 or mixed q, 4 rows per tile.
 // HELM_AMD_KERNEL = mfma | valu | generic restricts the choice (valu: no
 // matrix cores; generic: the element-wise kernel only).
@@ -214,7 +214,7 @@ void settle_fused(Plan& pl, int B, int Hkv) {
 
 // Rows, tiles and the split limits of a kernel choice.
 void plan_shape(Plan& pl, int G, int q_len, int D, int max_tok_per_page) {
-  pl.nw = pl.mfma ? mfma_waves() : kWaves;
+  pl.nw = pl.mfma && D == 128 ? mfma_waves() : kWaves;
   if (pl.mfma) {
     pl.gm = kMfmaRows;
     pl.rows = std::min(kMfmaRows, G * q_len);
@@ -231,7 +231,7 @@ void plan_shape(Plan& pl, int G, int q_len, int D, int max_tok_per_page) {
   // once per tile); HELM_AMD_ROW_WAVES=0 keeps one tile per workgroup
   // (HELM_AMD_CHUNK=16 keeps 16-row waves: chunk_mfma_kernel)
   pl.row_waves = (pl.mfma && pl.n_qtiles >= 2 && env_int("HELM_AMD_ROW_WAVES", 1))
-                     ? (env_int("HELM_AMD_CHUNK", 32) == 16 ? 1 : 2)
+                     ? (D == 128 && env_int("HELM_AMD_CHUNK", 32) == 16 ? 1 : 2)
                      : 0;
   if (pl.row_waves) pl.nw = kChunkStage;  // four waves per workgroup (see make_plan)
 }
@@ -312,9 +312,11 @@ int make_plan(Plan& pl, int kv_dtype, int q_dtype, int B, int Hq, int Hkv,
                 "query dtype must equal the KV dtype or be float32");
   const int G = Hq / Hkv;
   const int choice = kernel_choice();
-  const bool same16 = kv_dtype == q_dtype && kv_dtype != HELM_F32 && D == 128 && aligned16;
-  pl.mfma = (choice >= 2 && same16) ? 1 : 0;
-  pl.fast = (!pl.mfma && choice >= 1 && same16 && G <= 8) ? 1 : 0;
+  // D = 64 and 256 as D = 128: the matrix cores win from one token up (the
+  // figures are in attn_mfma.h and attn_chunk32.h); other head dims would pad
+  const bool same16 = kv_dtype == q_dtype && kv_dtype != HELM_F32 && aligned16;
+  pl.mfma = (choice >= 2 && same16 && (D == 64 || D == 128 || D == 256)) ? 1 : 0;
+  pl.fast = (!pl.mfma && choice >= 1 && same16 && D == 128 && G <= 8) ? 1 : 0;
   plan_shape(pl, G, q_len, D, max_tok_per_page);
   // chunk32 with eight waves (one workgroup of 256 query rows per CU) where a
   // KV head has at least 256 rows and the chunk attends over at least twice
@@ -322,7 +324,7 @@ int make_plan(Plan& pl, int kv_dtype, int q_dtype, int B, int Hq, int Hkv,
   // instead of once per 128 (512-token chunk over 32k: 0.43 -> 0.41 ms); a
   // first prompt chunk keeps four (its causal walks end earlier per
   // workgroup).  HELM_AMD_CHUNK_WAVES = 4 | 8 forces one.
-  if (pl.row_waves == 2) {
+  if (pl.row_waves == 2 && D == 128) {
     const int forced = env_int("HELM_AMD_CHUNK_WAVES", 0);
     const bool eight = forced ? forced == 8
                               : pl.n_qtiles >= 16 &&
@@ -336,7 +338,8 @@ int make_plan(Plan& pl, int kv_dtype, int q_dtype, int B, int Hq, int Hkv,
     // of LDS and 2 waves per SIMD let two share a CU): longer splits mean
     // fewer partials
     const int target =
-        env_int("HELM_AMD_WG_PER_CU", pl.row_waves && pl.nw == 4 ? 2 : 1) * device_cus();
+        env_int("HELM_AMD_WG_PER_CU", pl.row_waves && pl.nw == 4 && D <= 128 ? 2 : 1) *
+        device_cus();
     const double splits = std::max(1.0, target / units);
     pps = (int)std::ceil(std::max(1.0, avg_pages) / splits);
     pps = std::max(pps, min_pps(pl.bpp, pl.nw));
@@ -436,7 +439,7 @@ void fill_params(AttnParams& a, const Plan& pl, const void* q, void* out,
 // default) gives the same bits for the same inputs.
 void enable_claims(AttnParams& a, const Plan& pl, int B, int Hkv, char* ws) {
   const size_t tiles = (size_t)B * Hkv * pl.n_qtiles;
-  if (!pl.mfma || pl.row_waves || tiles * kClaimStride * 4 > kClaimRegionBytes ||
+  if (!pl.mfma || pl.row_waves || a.D != 128 || tiles * kClaimStride * 4 > kClaimRegionBytes ||
       !env_int("HELM_AMD_CLAIM", 0))
     return;
   a.dyn = 1;
@@ -444,6 +447,11 @@ void enable_claims(AttnParams& a, const Plan& pl, int B, int Hkv, char* ws) {
 }
 
 hipError_t dispatch(const LaunchSpec& s, hipStream_t st) {
+  if (s.mfma && s.p.D != 128) {
+    const bool bf = s.kv_dtype == HELM_BF16;
+    if (s.p.D == 64) return bf ? launch_attn_bf16_d64(s, st) : launch_attn_f16_d64(s, st);
+    return bf ? launch_attn_bf16_d256(s, st) : launch_attn_f16_d256(s, st);
+  }
   switch (s.kv_dtype) {
     case HELM_F16: return launch_attn_f16(s, st);
     case HELM_BF16: return launch_attn_bf16(s, st);
@@ -506,6 +514,38 @@ hipError_t dispatch_timed(const LaunchSpec& s, hipStream_t st) {
   return dispatch(s, st);
 }
 
+// launch_merge at the head dims with a merge of their own.  rows: few splits
+// per tile (query chunks), one thread per (row, column chunk) walking the
+// splits, 256 / (D / 4) rows per workgroup.
+template <typename TQ, int D>
+hipError_t launch_merge_dim(const LaunchSpec& s, bool rows, dim3 grid, hipStream_t st) {
+  constexpr int kRows = kThreads / (D / 4);
+  const dim3 rgrid(grid.x, (s.p.rows_per_tile + kRows - 1) / kRows);
+  if constexpr (D == 128) {
+    if (rows)
+      hipLaunchKernelGGL(merge_rows_d128_kernel<TQ>, rgrid, dim3(kThreads), 0, st, s.p);
+    else
+      hipLaunchKernelGGL(merge_splits_d128_kernel<TQ>, grid, dim3(kThreads), 0, st, s.p);
+  } else if (rows) {
+    hipLaunchKernelGGL((merge_rows_dim_kernel<TQ, D>), rgrid, dim3(kThreads), 0, st, s.p);
+  } else {
+    hipLaunchKernelGGL((merge_splits_dim_kernel<TQ, D>), grid, dim3(kThreads), 0, st, s.p);
+  }
+  return hipGetLastError();
+}
+
+template <typename TQ>
+hipError_t launch_merge_q(const LaunchSpec& s, int groups, dim3 grid, hipStream_t st) {
+  const bool rows = s.p.max_splits <= kMergeBatch && env_int("HELM_AMD_MERGE_ROWS", 1);
+  if (groups == 1) {
+    if (s.p.D == 128) return launch_merge_dim<TQ, 128>(s, rows, grid, st);
+    if (s.p.D == 64) return launch_merge_dim<TQ, 64>(s, rows, grid, st);
+    if (s.p.D == 256) return launch_merge_dim<TQ, 256>(s, rows, grid, st);
+  }
+  hipLaunchKernelGGL(merge_splits_kernel<TQ>, grid, dim3(kThreads), 0, st, s.p);
+  return hipGetLastError();
+}
+
 // Combines the split partials of every tile into the output (after the
 // split kernels, on the same stream).
 hipError_t launch_merge(const LaunchSpec& s, int B, int Hkv, hipStream_t st) {
@@ -514,51 +554,12 @@ hipError_t launch_merge(const LaunchSpec& s, int B, int Hkv, hipStream_t st) {
   const int chunks = (s.p.D % 4 == 0) ? s.p.D / 4 : s.p.D;
   const int groups = std::max(1, std::min(env_int("HELM_AMD_MERGE_GROUPS", 1), chunks));
   const dim3 grid(B * Hkv * s.p.n_qtiles, s.p.rows_per_tile, groups);
-  // few splits per tile (query chunks): one thread per (row, column chunk)
-  // walking the splits, eight rows per workgroup
-  if (s.p.D == 128 && groups == 1 && s.p.max_splits <= kMergeBatch &&
-      env_int("HELM_AMD_MERGE_ROWS", 1)) {
-    const dim3 rgrid(B * Hkv * s.p.n_qtiles, (s.p.rows_per_tile + 7) / 8);
-    switch (s.q_dtype) {
-      case HELM_F16:
-        hipLaunchKernelGGL(merge_rows_d128_kernel<f16_t>, rgrid, dim3(kThreads), 0, st, s.p);
-        return hipGetLastError();
-      case HELM_BF16:
-        hipLaunchKernelGGL(merge_rows_d128_kernel<bf16_t>, rgrid, dim3(kThreads), 0, st, s.p);
-        return hipGetLastError();
-      case HELM_F32:
-        hipLaunchKernelGGL(merge_rows_d128_kernel<float>, rgrid, dim3(kThreads), 0, st, s.p);
-        return hipGetLastError();
-      default: return hipErrorInvalidValue;
-    }
-  }
-  if (s.p.D == 128 && groups == 1) {
-    switch (s.q_dtype) {
-      case HELM_F16:
-        hipLaunchKernelGGL(merge_splits_d128_kernel<f16_t>, grid, dim3(kThreads), 0, st, s.p);
-        return hipGetLastError();
-      case HELM_BF16:
-        hipLaunchKernelGGL(merge_splits_d128_kernel<bf16_t>, grid, dim3(kThreads), 0, st, s.p);
-        return hipGetLastError();
-      case HELM_F32:
-        hipLaunchKernelGGL(merge_splits_d128_kernel<float>, grid, dim3(kThreads), 0, st, s.p);
-        return hipGetLastError();
-      default: return hipErrorInvalidValue;
-    }
-  }
   switch (s.q_dtype) {
-    case HELM_F16:
-      hipLaunchKernelGGL(merge_splits_kernel<f16_t>, grid, dim3(kThreads), 0, st, s.p);
-      break;
-    case HELM_BF16:
-      hipLaunchKernelGGL(merge_splits_kernel<bf16_t>, grid, dim3(kThreads), 0, st, s.p);
-      break;
-    case HELM_F32:
-      hipLaunchKernelGGL(merge_splits_kernel<float>, grid, dim3(kThreads), 0, st, s.p);
-      break;
+    case HELM_F16: return launch_merge_q<f16_t>(s, groups, grid, st);
+    case HELM_BF16: return launch_merge_q<bf16_t>(s, groups, grid, st);
+    case HELM_F32: return launch_merge_q<float>(s, groups, grid, st);
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 // ---- page append kernel -----------------------------------------------------
@@ -1183,6 +1184,14 @@ int helm_paged_decode_attn(const void* q, void* out, const void* k_pool,
     size_plan(pl, B, Hkv, D);
     settle_fused(pl, B, Hkv);
   }
+  if (ws_bytes < pl.total() && pl.mfma && D != 128) {
+    // a workspace below the matrix-core plan's need (its tiles hold up to 16
+    // rows, and more splits): the element-wise kernel's plan may still fit
+    rc = make_plan(pl, kv_dtype, q_dtype, B, Hq, Hkv, q_len, D, page_size, max_pages, avg,
+                   pages_per_split, false);
+    if (rc != HELM_OK) return rc;
+    compact = false;
+  }
   if (ws_bytes < pl.total())
     return fail(HELM_E_WORKSPACE,
                 "workspace too small: need " + std::to_string(pl.total()));
@@ -1649,7 +1658,7 @@ static int paged_attn_seqs(helm_engine* eng, const void* q, void* out, int B, in
   if (rc != HELM_OK) return rc;
   if (app) {
     // the token writes run inside the matrix-core decode kernel only
-    if (!(pl.mfma && !pl.row_waves && q_len == 1 && D == 128 && eb == 2))
+    if (!(pl.mfma && !pl.row_waves && q_len == 1 && D == 128))
       return fail(HELM_E_UNSUPPORTED, "token writes need the matrix-core decode kernel");
     for (int b = 0; b < B; ++b) {
       const helm_append_seg& a = app[b];

@@ -1,0 +1,103 @@
+"""The matrix-core kernels at head dims 64 and 256 against the float64 oracle.
+
+The sizes sit at the edges of the kernels' tiles: one row, 16-row decode tiles
+(full, remainder), 32-row chunk waves and 128-row workgroups, 16-token blocks,
+four-block stages, 64-page record windows; one or several splits and both
+merges.  Tolerances: the output's own rounding (half an ulp of the largest
+element, |out| < 4: 2^-9 relative in bf16, 2^-12 in f16) and the weights' hi +
+lo split (2^-16 of sum |w v|, below it): 1e-2 (bf16) and 2e-3 (f16) absolute.
+"""
+import math
+
+import pytest
+import torch
+
+from helm_amd import workloads as W
+from helm_amd.paged import paged_decode_attention
+from helm_amd.runtime.kv_cache import KVPage, perform_streaming_attention
+from oracle import attention as A
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+TOL = {torch.float16: 2e-3, torch.bfloat16: 1e-2}
+
+
+def _pages(K, V, sizes):
+    pages, t = [], 0
+    for i, n in enumerate(sizes):
+        k, v = (x[:, :, t:t + n].contiguous().to(DEV) for x in (K, V))
+        pages.append(KVPage(page_id=i, layer_id=0, start_token=t, used_tokens=n,
+                            capacity_tokens=n, k_tensor=k, v_tensor=v, device=k.device,
+                            state="GPU"))
+        t += n
+    return pages
+
+
+def _mask(kind, S, T, dtype):
+    """(the additive mask as given, what the oracle adds) of a later chunk."""
+    if kind in ("none", "causal"):
+        return None
+    pos = torch.arange(T - S, T)[:, None]
+    key = torch.arange(T)[None, :]
+    seen = key <= pos
+    if kind == "window":
+        seen = seen & (key > pos - max(1, T // 3))
+    low = torch.finfo(dtype).min
+    m = torch.zeros(S, T, dtype=dtype).masked_fill_(~seen, low)
+    if kind == "first_row_masked":      # one row with no visible key: equal weights
+        m[0] = low
+    return m[None, None]
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,S,sizes", [
+    (4, 4, 1, [1]),                      # one row, one token
+    (6, 2, 1, [16, 16, 5]),              # a partial decode tile, a partial block
+    (32, 2, 1, [16] * 70 + [3]),         # a full 16-row tile, past one record window
+    (40, 2, 1, [64, 64, 17]),            # more than one tile per KV head
+    (4, 2, 17, [16, 16, 11]),            # 34 chunk rows: a full wave and two rows
+    (14, 2, 19, [64, 64, 64, 30]),       # 133 rows: a workgroup and five rows
+    (4, 1, 150, [16] * 68 + [7]),        # several workgroups, past one record window
+])
+@pytest.mark.parametrize("kind,cap", [("none", None), ("causal", None), ("window", None),
+                                      ("window", 5.0), ("first_row_masked", None)])
+def test_streaming_matches_fp64(D, dtype, Hq, Hkv, S, sizes, kind, cap):
+    T = sum(sizes)
+    if kind == "causal" and S == 1 or kind == "none" and S > 1 or T < S and kind != "causal":
+        pytest.skip("no such call")
+    g = torch.Generator().manual_seed(D + 7 * S + T)
+    K = torch.randn(1, Hkv, T, D, generator=g).to(dtype)
+    V = torch.randn(1, Hkv, T, D, generator=g).to(dtype)
+    q = (1.5 * torch.randn(1, Hq, S, D, generator=g)).to(dtype)
+    m = _mask(kind, S, T, dtype)
+    out = perform_streaming_attention(q.to(DEV), _pages(K, V, sizes), softcap=cap,
+                                      attention_mask=None if m is None else m.to(DEV))
+    ref_m = m
+    if kind == "causal":
+        ref_m = torch.zeros(1, 1, S, T).masked_fill_(
+            torch.arange(T)[None, :] > torch.arange(S)[:, None], -math.inf)
+    ref = A.attention_fp64_batched(q[0], K[0], V[0], softcap=cap,
+                                   mask=None if ref_m is None else ref_m[0])
+    err = (out[0].double().cpu() - ref).abs().max().item()
+    assert err <= TOL[dtype], err
+
+
+@pytest.mark.parametrize("merge", ["fused", "kernel"])
+@pytest.mark.parametrize("D,P", [(64, 16), (64, 64), (256, 16), (256, 64)])
+@pytest.mark.parametrize("lens,pps", [([1, 15, 16, 17], 0), ([3001], 0), ([3001], 1),
+                                      ([700, 64, 2049], 3)])
+def test_pool_decode_matches_fp64(D, P, lens, pps, merge, monkeypatch):
+    monkeypatch.setenv("HELM_AMD_MERGE", merge)
+    for dtype in (torch.bfloat16, torch.float16):
+        w = W.Workload("dims", len(lens), 10, 2, D, dtype, T=max(lens), page_size=P)
+        case = W.make_pool_case(w, seed=D + P, device=DEV, lens=lens)
+        out = paged_decode_attention(case["q"], case["k_pool"], case["v_pool"], case["table"],
+                                     case["lens"], max_pages=case["max_pages"],
+                                     pages_per_split=pps)
+        for b, T in enumerate(lens):
+            rows = case["pool"][case["table"][b, :case["n_pages"][b]].long()].cpu()
+            kv = rows.permute(1, 2, 0, 3, 4).reshape(2, w.Hkv, -1, D)[:, :, :T]
+            ref = A.attention_fp64_batched(case["q"][b].cpu(), kv[0], kv[1])
+            err = (out[b].double().cpu() - ref).abs().max().item()
+            assert err <= TOL[dtype], (dtype, b, err)
