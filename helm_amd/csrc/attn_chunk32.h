@@ -306,20 +306,57 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   };
 
   // additive mask of row jr for the step of blocks bp, bp + 1 of a stage:
-  // tokens 8hh .. 8hh + 7 of each block, bounded by its valid tokens
-  float mk_next[16];
+  // tokens 8hh .. 8hh + 7 of each block, bounded by its valid tokens, as
+  // loaded: words 0 .. 7 of a block for an fp32 mask, 0 .. 3 (two tokens each)
+  // for a 16-bit one.  A whole block's tokens are 16-byte loads at the mask's
+  // own alignment; a partial block's go one by one, the index clamped to its
+  // last valid token.  Element loads of every block, 16 per step, had bound the
+  // masked chunk, and a zero mask was added all the same: bf16 512 over 8,192
+  // tokens under a 4,096-token window, 32 / 8 heads, 187 -> 121 us; D = 256, 512
+  // over 4,700, soft-capped, 203 -> 106 us (tanhf per score was the rest).
+  // (Whole-vector values: element stores from several branches would put the
+  // words in scratch memory.)
+  mf_u32x8 mk_next[2];
+  auto load_block_mask = [&](int nt, int tok0) -> mf_u32x8 {
+    const MaskRow mb = mrow + tok0;
+    if (__builtin_expect(nt == kBlockTok, 1)) {
+      const char* src = (mb + 8 * hh).base;
+      const mf_u32x4 a = load16_any(src);
+      const mf_u32x4 c = p.mask_dt == HELM_F32 ? load16_any(src + 16) : mf_u32x4{0u, 0u, 0u, 0u};
+      return mf_u32x8{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+    }
+    if (nt == 0) return mf_u32x8{0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+    auto f32 = [&](int i) -> uint32_t {
+      return mb.template bits<false>(min(8 * hh + i, nt - 1));
+    };
+    auto h16 = [&](int i) -> uint32_t {
+      return mb.template bits<true>(min(8 * hh + i, nt - 1)) |
+             (uint32_t)mb.template bits<true>(min(8 * hh + i + 1, nt - 1)) << 16;
+    };
+    if (p.mask_dt == HELM_F32)
+      return mf_u32x8{f32(0), f32(1), f32(2), f32(3), f32(4), f32(5), f32(6), f32(7)};
+    return mf_u32x8{h16(0), h16(2), h16(4), h16(6), 0u, 0u, 0u, 0u};
+  };
   auto load_step_mask = [&](const int (&ntok)[SB], const int (&tok0)[SB], int bp) {
     if constexpr (kMask) {
-      // (plain loads: the row differs between lanes; past the block's last
-      // valid token the index is clamped to it)
+      mk_next[0] = load_block_mask(ntok[bp], tok0[bp]);
+      mk_next[1] = load_block_mask(ntok[bp + 1], tok0[bp + 1]);
+    }
+  };
+  // any bit of the step's mask words set (a zero mask adds nothing to any score)
+  auto mask_bits = [&](const mf_u32x8& a, const mf_u32x8& b) -> uint32_t {
+    const mf_u32x8 w = a | b;   // (a 16-bit mask's last four words are zero)
+    return w[0] | w[1] | w[2] | w[3] | w[4] | w[5] | w[6] | w[7];
+  };
+  // a block's eight mask values in fp32
+  auto mask_values = [&](const mf_u32x8& w, float* mk) {
+    if (p.mask_dt == HELM_F32) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int nt = ntok[bp + u];
-        const int last = max(nt - 1, 0);
-        const MaskRow mb = mrow + tok0[bp + u];
+      for (int i = 0; i < 8; ++i) mk[i] = __uint_as_float(w[i]);
+    } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) mk_next[8 * u + i] = nt > 0 ? mb[min(8 * hh + i, last)] : 0.f;
-      }
+      for (int i = 0; i < 8; ++i)
+        mk[i] = mrow.template widen<true>((i & 1) ? w[i >> 1] >> 16 : w[i >> 1] & 0xffffu);
     }
   };
 
@@ -394,21 +431,24 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
         return false;
       };
       // logits, online softmax and P . V of one step
-      auto finish = [&](int bp, const mf_f32x16& sc, const float* mk) {
+      auto finish = [&](int bp, const mf_f32x16& sc, bool add_mask, const float (&mk)[16]) {
         const int nt0 = ntok_c[bp], nt1 = ntok_c[bp + 1];
         float x[16];
+        if constexpr (kCap) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float val;
-          if constexpr (kCap)
-            val = tanhf(sc[r] * scale * inv_cap) * cap2;
-          else
-            val = sc[r] * scale2;
-          // finfo.min masks stay finite, as in natural units (a row masked
-          // everywhere gets equal weights, as HELM's loop gives it)
-          if constexpr (kMask) val = fmaxf(fmaf(mk[r], kLog2E, val), -__FLT_MAX__);
-          x[r] = val;
+          for (int r = 0; r < 16; ++r) x[r] = sc[r];
+          softcap_scores<16>(x, scale * inv_cap, cap2);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) x[r] = sc[r] * scale2;
         }
+        // finfo.min masks stay finite, as in natural units (a row masked
+        // everywhere gets equal weights, as HELM's loop gives it)
+        if constexpr (kMask)
+          if (add_mask)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+              x[r] = fmaxf(fmaf(mk[r], kLog2E, x[r]), -__FLT_MAX__);
         // the per-token limits, only where a step reaches them (uniform tests):
         // the causal limit when a block's last token is past the wave's first
         // query position, the valid-token limit when a block is partial
@@ -488,10 +528,10 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
 #pragma unroll
         for (int bp = 0; bp < SB; bp += 2) {     // the step's blocks bp, bp + 1
           // the mask of the next step is loaded now, one step ahead of its use
-          float mk[16];
+          mf_u32x8 mw0, mw1;
           if constexpr (kMask) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mk[r] = mk_next[r];
+            mw0 = mk_next[0];
+            mw1 = mk_next[1];
             if (bp + 2 < SB)
               load_step_mask(ntok_c, tok0_c, bp + 2);
             else if (st + 1 < nstage)
@@ -501,15 +541,22 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
           // masked, a step whose every mask value is <= -1e30 while every
           // row's max is already above -1e20 adds exactly nothing (each
           // weight underflows to 0 and the max stays)
+          float mk[16];
+          bool add_mask = false;
           if constexpr (kMask) {
-            float mm = mk[0];
+            add_mask = __builtin_amdgcn_ballot_w64(mask_bits(mw0, mw1) != 0u) != 0;
+            if (add_mask) {
+              mask_values(mw0, mk);
+              mask_values(mw1, mk + 8);
+              float mm = mk[0];
 #pragma unroll
-            for (int r = 1; r < 16; ++r) mm = fmaxf(mm, mk[r]);
-            if (!__builtin_amdgcn_ballot_w64(mm > -1e30f) &&
-                !__builtin_amdgcn_ballot_w64(m <= -1e20f))
-              continue;
+              for (int r = 1; r < 16; ++r) mm = fmaxf(mm, mk[r]);
+              if (!__builtin_amdgcn_ballot_w64(mm > -1e30f) &&
+                  !__builtin_amdgcn_ballot_w64(m <= -1e20f))
+                continue;
+            }
           }
-          finish(bp, qk(bp), mk);
+          finish(bp, qk(bp), add_mask, mk);
         }
       }
     }

@@ -153,6 +153,46 @@ __device__ __forceinline__ typename VRow<D>::type buf_load_vrow_nt(__amdgpu_buff
   }
 }
 
+// 16 bytes at any alignment (one load: the target takes unaligned vector loads).
+__device__ __forceinline__ mf_u32x4 load16_any(const char* p) {
+  struct __attribute__((packed)) Any { mf_u32x4 v; };
+  return reinterpret_cast<const Any*>(p)->v;
+}
+
+// x = cap tanh(x k) with k = scale / cap and cap in the caller's log units, for
+// the N scores of a lane.  Logits far below the cap (|x k| <= 2^-2.5 for every
+// score of the wave, |logit| <= 8.8 at a cap of 50: the usual case) take the
+// odd Taylor polynomial of tanh through y^7, whose first left-out term is below
+// 2.1e-8 of the result there, an eighth of an fp32 ulp; up to |x k| <= 1/2 the
+// one through y^13 (8.9e-8); any other step tanhf.
+template <int N>
+__device__ __forceinline__ void softcap_scores(float (&x)[N], float k, float cap) {
+  float top = fabsf(x[0]);
+#pragma unroll
+  for (int r = 1; r < N; ++r) top = fmaxf(top, fabsf(x[r]));
+  top *= k;
+  constexpr float c1 = -1.f / 3.f, c2 = 2.f / 15.f, c3 = -17.f / 315.f, c4 = 62.f / 2835.f,
+                  c5 = -1382.f / 155925.f, c6 = 21844.f / 6081075.f;
+  const float kc = k * cap;
+  if (__builtin_expect(!__builtin_amdgcn_ballot_w64(!(top <= 0.1767767f)), 1)) {
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      const float y = x[r] * k, z = y * y;
+      x[r] = x[r] * kc * fmaf(z, fmaf(z, fmaf(z, c3, c2), c1), 1.f);
+    }
+  } else if (!__builtin_amdgcn_ballot_w64(!(top <= 0.5f))) {
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      const float y = x[r] * k, z = y * y;
+      const float h = fmaf(z, fmaf(z, fmaf(z, c6, c5), c4), c3);
+      x[r] = x[r] * kc * fmaf(z, fmaf(z, fmaf(z, h, c2), c1), 1.f);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < N; ++r) x[r] = tanhf(x[r] * k) * cap;
+  }
+}
+
 // LDS transpose read of 16-bit elements (ds_read_b64_tr_b16): within each
 // 16-lane group, lane c = 4a + b receives element b of the 8 bytes that
 // lanes a, a + 4, a + 8 and a + 12 address, in that order.
@@ -285,13 +325,13 @@ __device__ __forceinline__ void mfma_logits(mf_f32x4 sc, const float (&mk)[4], i
                                             float scale, float cap, float inv_cap, int s_vis,
                                             int q4, float (&x)[4]) {
 #pragma unroll
+  for (int r = 0; r < 4; ++r) x[r] = kCap ? sc[r] : sc[r] * scale;
+  if constexpr (kCap) softcap_scores<4>(x, scale * inv_cap, cap);
+#pragma unroll
   for (int r = 0; r < 4; ++r) {
-    float val = sc[r] * scale;
-    if constexpr (kCap) val = tanhf(val * inv_cap) * cap;
-    if constexpr (kMask) val += mk[r];
+    if constexpr (kMask) x[r] += mk[r];
     if constexpr (kCausal)
-      if (tok0 + 4 * r + q4 > s_vis) val = -INFINITY;
-    x[r] = val;
+      if (tok0 + 4 * r + q4 > s_vis) x[r] = -INFINITY;
   }
   if (ntok < kBlockTok) {
 #pragma unroll
