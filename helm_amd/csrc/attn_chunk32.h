@@ -88,6 +88,22 @@ __device__ __forceinline__ void buf_load16_lds(__amdgpu_buffer_rsrc_t r, void* l
                                            off, 0, 0, 0);
 }
 
+// The workgroup's block of query rows.  Under a causal limit a block's walk
+// grows with its index; p.qb_round > 0 (blocks per head that the device's CUs
+// take in one round of workgroups, in launch order) hands the blocks out
+// longest first, every second round in reverse, so that the workgroups that
+// share a CU add up to about the same walk and the shortest come last (bf16
+// first prompt of 2,048, 40 / 8 heads: in index order 83, longest first 65 us;
+// 32 / 32 heads: 67, longest first 61.5, with the reversal 59.6).
+__device__ __forceinline__ int query_block(const AttnParams& p) {
+  const int j = blockIdx.y / p.Hkv;
+  if (p.qb_round <= 0) return j;
+  const int n = gridDim.y / p.Hkv;
+  const int r = j / p.qb_round, first = r * p.qb_round;
+  const int last = min(n, first + p.qb_round) - 1;
+  return n - 1 - ((r & 1) ? last - (j - first) : j);
+}
+
 // NW waves per workgroup (4: two workgroups per CU; 8: one, which halves the
 // stage loads per query row), 32 query rows each.
 template <typename T, class Src, int FEAT, int NW, int D>
@@ -126,7 +142,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   const int split_local = blockIdx.x;
   const int hk = blockIdx.y % p.Hkv;
   const int n32 = (p.n_qtiles + 1) / 2;                 // 32-row groups of the head
-  const int wt = (blockIdx.y / p.Hkv) * NW + wave;
+  const int wt = query_block(p) * NW + wave;
   const bool wave_rows = wt < n32;
   const int wtc = wave_rows ? wt : n32 - 1;
   const int b = blockIdx.z;
@@ -370,7 +386,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   // add nothing for any of its rows (a causal call lists a launch's pages in
   // token order, so tokens only grow along the walk), and the walk ends
   // there (uniform across the workgroup)
-  const int qrow_end = min(G * S, (int)(blockIdx.y / p.Hkv + 1) * NW * kChunk32Rows);
+  const int qrow_end = min(G * S, (query_block(p) + 1) * NW * kChunk32Rows);
   const int s_last_wg = (qrow_end - 1) / G + coff;
   bool done = false;
   // stage st (view slot K = st % 2) computes from `cur` while the loads of
@@ -380,7 +396,9 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
     const int (&ntok_c)[SB] = vnt[K];
     const int (&tok0_c)[SB] = vt0[K];
     if constexpr (kCausal) {
-      if (tok0_c[0] > s_last_wg) {
+      // (an empty block, past the used tokens of a page shorter than the
+      // longest, says nothing: the next page's tokens may lie before its offset)
+      if (ntok_c[0] > 0 && tok0_c[0] > s_last_wg) {
         __builtin_amdgcn_s_waitcnt(0x0F70);   // this stage's loads land before the exit
         done = true;
         return;

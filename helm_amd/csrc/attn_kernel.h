@@ -490,6 +490,7 @@ struct AttnParams {
   int fused;          // 1: the last split of a tile merges in-kernel
   int row_waves;      // query chunks: 16-row tiles per wave (1 or 2; 0: decode kernel)
   int direct_out;     // 1: the call has one split; the chunk kernel writes the output
+  int qb_round;       // causal query chunks: see query_block (attn_chunk32.h); 0: off
   int bpp_log2;       // log2 of bpp when bpp is a power of two, else -1
   // profiling (helm_profile_workgroup_stamps): per workgroup of the decode
   // kernel {start, page loop end, end, XCD << 32 | HW_ID}; null: off

@@ -295,11 +295,45 @@ int balanced_pps(double pages, double units, int target, int lo_pps, int max_pps
   return best_pps;
 }
 
+// Pages per split of a query chunk on the 32-row kernel.  The splits are
+// numbered so that the estimate of the call is least: the work, the longest
+// split's walk or the share of the busiest CU, and with more than one split
+// the fp32 partials' way to memory and back and the merge's launch.  walk: the
+// mean share of the pages a query block walks (a causal first prompt: about
+// half).  Measured per 64-token stage (one workgroup alone / per workgroup on
+// a full CU, us): D = 128 four waves 2.0 / 1.6, eight waves 2.3; D = 64
+// 1.6 / 1.0; D = 256 3.3.  A split length from the number of workgroups alone gave
+// 480-workgroup prompts a second split of a few pages and its partials (f16
+// 40 heads, 1,500 tokens: 97 us, one split 47; bf16 8 heads, 4,000 tokens: 85,
+// now 71).
+int chunk_pps(const Plan& pl, int D, double units, double rows, double pages, double walk) {
+  const double alone = D == 256 ? 3.3 : D == 64 ? 1.6 : pl.nw == 8 ? 2.3 : 2.0;
+  const double full = D == 256 ? 3.3 : D == 64 ? 1.0 : pl.nw == 8 ? 2.3 : 1.6;
+  constexpr double kMergeUs = 6.0, kPartialBytesPerUs = 5e6;
+  const double P = std::max(1.0, pages);
+  const double cus = device_cus();
+  int best_pps = (int)std::ceil(P);
+  double best = -1.0;
+  for (int s = 1; s <= 64 && s <= P; ++s) {
+    const int pps = (int)std::ceil(P / s);
+    const double n = std::ceil(P / pps);
+    const double stages = pps * (double)pl.bpp / kChunkStage;
+    const double share = walk > 0.75 ? std::ceil(units * n / cus) : units * n * walk / cus;
+    double us = std::max(stages * alone, share * stages * full);
+    if (n > 1) us += kMergeUs + n * rows * D * 8.0 / kPartialBytesPerUs;
+    if (best < 0.0 || us < best) {
+      best = us;
+      best_pps = pps;
+    }
+  }
+  return best_pps;
+}
+
 // work_pages: pages one (sequence, head, tile) walks on average; max_pages:
 // the longest sequence (bounds the split count).
 int make_plan(Plan& pl, int kv_dtype, int q_dtype, int B, int Hq, int Hkv,
               int q_len, int D, int max_tok_per_page, int max_pages,
-              double avg_pages, int pps_req, bool aligned16) {
+              double avg_pages, int pps_req, bool aligned16, int causal) {
   if (Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0)
     return fail(HELM_E_INVALID, "Hq must be a positive multiple of Hkv");
   if (D <= 0 || D > 256)
@@ -332,6 +366,11 @@ int make_plan(Plan& pl, int kv_dtype, int q_dtype, int B, int Hq, int Hkv,
     if (eight) pl.nw = 8;
   }
   int pps = pps_req > 0 ? pps_req : env_int("HELM_AMD_PPS", 0);
+  if (pps <= 0 && pl.row_waves == 2 && env_int("HELM_AMD_WG_PER_CU", 0) <= 0) {
+    const double tokens = std::max(1.0, avg_pages * max_tok_per_page);
+    const double walk = causal ? std::min(1.0, (causal + 0.5 * q_len) / tokens) : 1.0;
+    pps = chunk_pps(pl, D, (double)B * Hkv * pl.qblocks(), (double)B * Hq * q_len, avg_pages, walk);
+  }
   if (pps <= 0) {
     const double units = (double)B * Hkv * pl.qblocks();
     // one workgroup per CU (two for the four-wave chunk kernels, whose 64 KiB
@@ -402,6 +441,9 @@ void fill_params(AttnParams& a, const Plan& pl, const void* q, void* out,
   a.n_qtiles = pl.n_qtiles;
   a.row_waves = pl.row_waves;
   a.direct_out = pl.direct;
+  // (one split: with several, every walk is a split's length at most)
+  a.qb_round =
+      causal && pl.row_waves == 2 && pl.direct ? std::max(1, device_cus() / (Hkv * B)) : 0;
   a.scale = scale;
   a.softcap = softcap;
   a.mask = mask;
@@ -1159,7 +1201,7 @@ int helm_paged_decode_attn(const void* q, void* out, const void* k_pool,
   const double avg = total_pages > 0 ? (double)total_pages / B : max_pages;
   Plan pl{};
   int rc = make_plan(pl, kv_dtype, q_dtype, B, Hq, Hkv, q_len, D, page_size,
-                     max_pages, avg, pages_per_split, al);
+                     max_pages, avg, pages_per_split, al, 0);
   if (rc != HELM_OK) return rc;
   // the sequences' lengths on the host (a batch on the decode kernel): the
   // split length from every sequence's page count and a grid of exactly
@@ -1188,7 +1230,7 @@ int helm_paged_decode_attn(const void* q, void* out, const void* k_pool,
     // a workspace below the matrix-core plan's need (its tiles hold up to 16
     // rows, and more splits): the element-wise kernel's plan may still fit
     rc = make_plan(pl, kv_dtype, q_dtype, B, Hq, Hkv, q_len, D, page_size, max_pages, avg,
-                   pages_per_split, false);
+                   pages_per_split, false, 0);
     if (rc != HELM_OK) return rc;
     compact = false;
   }
@@ -1456,7 +1498,7 @@ int helm_stream_attn(helm_engine* eng, const void* q, void* out, int B,
   }
   Plan pl{};
   int rc = make_plan(pl, kv_dtype, q_dtype, B, Hq, Hkv, q_len, D, max_tok,
-                     std::max(max_pages, 1), (double)n_all / B, 0, al);
+                     std::max(max_pages, 1), (double)n_all / B, 0, al, causal);
   if (rc != HELM_OK) return rc;
   if (n_host) {
     // every launch owns whole splits; keep the call within the split limit
@@ -1654,7 +1696,7 @@ static int paged_attn_seqs(helm_engine* eng, const void* q, void* out, int B, in
                   (D * qb) % 16 == 0;
   Plan pl{};
   int rc = make_plan(pl, kv_dtype, q_dtype, B, Hq, Hkv, q_len, D, page_tokens,
-                     std::max(max_pages, 1), (double)all_pages / B, 0, al);
+                     std::max(max_pages, 1), (double)all_pages / B, 0, al, causal);
   if (rc != HELM_OK) return rc;
   if (app) {
     // the token writes run inside the matrix-core decode kernel only

@@ -101,3 +101,21 @@ def test_pool_decode_matches_fp64(D, P, lens, pps, merge, monkeypatch):
             ref = A.attention_fp64_batched(case["q"][b].cpu(), kv[0], kv[1])
             err = (out[b].double().cpu() - ref).abs().max().item()
             assert err <= TOL[dtype], (dtype, b, err)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("Hq,Hkv,S", [(32, 32, 1300), (40, 8, 1000), (8, 8, 129)])
+def test_first_prompt_block_order(D, Hq, Hkv, S, monkeypatch):
+    """One causal split whose blocks of query rows are handed out longest
+    first, every second round of workgroups reversed: 11 blocks per head in
+    rounds of 8, 40 in rounds of 32, two in one round; every row once."""
+    monkeypatch.setenv("HELM_AMD_PPS", "4096")
+    g = torch.Generator().manual_seed(S + D)
+    K = torch.randn(1, Hkv, S, D, generator=g).to(torch.bfloat16)
+    V = torch.randn(1, Hkv, S, D, generator=g).to(torch.bfloat16)
+    q = (1.5 * torch.randn(1, Hq, S, D, generator=g)).to(torch.bfloat16)
+    out = perform_streaming_attention(q.to(DEV), _pages(K, V, [S // 3, S - S // 3]))
+    causal = torch.zeros(1, S, S).masked_fill_(
+        torch.arange(S)[None, :] > torch.arange(S)[:, None], -math.inf)
+    ref = A.attention_fp64_batched(q[0], K[0], V[0], mask=causal)
+    assert (out[0].double().cpu() - ref).abs().max().item() <= TOL[torch.bfloat16]
