@@ -1246,6 +1246,107 @@ def _decode_args():
     return a
 
 
+_NO_MASK = (0, 0, 0, _native.HELM_F32)
+
+
+def _decode_mask_args(m: torch.Tensor, device, B: int, Hq: int, t_max: int):
+    """(address, batch stride, head stride, element type) of a decode mask the
+    kernel reads as given, or None."""
+    code = _MASK_CODES.get(m.dtype)
+    mshape = m.shape
+    if (code is None or m.device != device or len(mshape) != 4
+            or mshape[0] not in (1, B) or mshape[1] not in (1, Hq) or mshape[2] != 1
+            or mshape[3] < t_max):
+        return None
+    mst = m.stride()
+    if mst[3] != 1:
+        return None
+    return (m.data_ptr(), mst[0] if mshape[0] > 1 else 0, mst[1] if mshape[1] > 1 else 0, code)
+
+
+def _decode_operands_plain(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """True when one native decode call can take the step's query and write its
+    tokens: 16-bit tensors of one dtype on a HIP device, D = 128, one 16-row
+    tile per KV head, dense 16-byte-aligned rows, and no environment switch
+    that asks for another route."""
+    B, Hq, S, D = q.shape
+    if (q.dtype not in _KV16 or S != 1 or D != 128 or B > _native.DECODE_MAX_SEQS
+            or not q.is_cuda or k.dtype is not q.dtype or v.dtype is not q.dtype
+            or not q.is_contiguous()):
+        return False
+    kB, Hkv, kS, _ = k.shape
+    ks, vs = k.stride(), v.stride()
+    if (Hq > 16 * Hkv                           # more than one 16-row tile per KV head
+            or kB < B or kS != 1 or ks[3] != 1 or vs[3] != 1 or ks[1] != vs[1]
+            or (ks[1] * 2) % 16
+            or (k.data_ptr() | v.data_ptr() | q.data_ptr() | (ks[0] * 2) | (vs[0] * 2)) % 16):
+        return False
+    return not (check_records_enabled()
+                or _env_get("HELM_AMD_FAST_DECODE") == "0"
+                or _env_get("HELM_AMD_FUSED_APPEND") == "0"
+                or _env_get("HELM_AMD_KERNEL") not in (None, "", "auto", "mfma"))
+
+
+def _decode_contiguous_fast(kvcms, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+                            layer_idx: int, scale: float,
+                            attention_mask: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """The decode step over contiguous buffers in one native call
+    (helm_decode_step): the attention kernel writes each item's token into its
+    buffer's last virtual page itself, which saves the append launch, and the
+    arguments go into this thread's block (four sequences of 8,200 tokens, 40 /
+    8 heads under a bf16 mask: 39.6 -> 27.1 us per step of one layer).  Every
+    item a KVCacheManager with room for the token, no write of its own queued,
+    and buffers of the query's dtype and device.  Returns None, with nothing
+    changed, when any of that does not hold."""
+    if not _decode_operands_plain(q, k, v):
+        return None
+    B, Hq, _, D = q.shape
+    Hkv = k.shape[1]
+    device, dtype = q.device, q.dtype
+    conts, t_max = [], 0
+    for kvcm in kvcms:
+        cont = kvcm._cont if type(kvcm) is KVCacheManager else None
+        n = kvcm.cont_seq_len
+        if (cont is None or n >= cont.capacity or not cont.aligned16 or kvcm._appends.rows
+                or layer_idx not in kvcm.cont_K):
+            return None
+        a = cont.arena
+        if a.dtype is not dtype or a.device != device or a.shape[2] != Hkv or a.shape[4] != D:
+            return None
+        conts.append((cont, n + 1))
+        t_max = max(t_max, n + 1)
+    if len(conts) != B or (B > 1 and len({id(c) for c, _ in conts}) != B):
+        return None
+    margs = _NO_MASK
+    if attention_mask is not None:
+        margs = _decode_mask_args(attention_mask, device, B, Hq, t_max)
+        if margs is None:
+            return None
+    mptr, mbs, mhs, mask_code = margs
+    _, buf, addr = _decode_args()
+    ks, vs = k.stride(), v.stride()
+    kp, vp, ks0, vs0, hs = k.data_ptr(), v.data_ptr(), ks[0] * 2, vs[0] * 2, ks[1]
+    u64, i64, i32 = _DA_U64.pack_into, _DA_I64.pack_into, _DA_I32.pack_into
+    for b, (cont, n) in enumerate(conts):
+        u64(buf, _DA_PAGES + 8 * b, cont.records_ptr(layer_idx))
+        u64(buf, _DA_TOKK + 8 * b, kp + b * ks0)
+        u64(buf, _DA_TOKV + 8 * b, vp + b * vs0)
+        i64(buf, _DA_TOKHS + 8 * b, hs)
+        i32(buf, _DA_NPAGES + 4 * b, -(-n // ContiguousKV.BLOCK))
+        i32(buf, _DA_TOKENS + 4 * b, n)
+    out = torch.empty_like(q)
+    _DA_HEAD.pack_into(buf, 0, q.data_ptr(), out.data_ptr(), mptr, _engine.stream_ptr(device),
+                       mbs, mhs, 0)
+    _DA_TAIL.pack_into(buf, _DA_TAIL_OFF, B, Hq, Hkv, D, ContiguousKV.BLOCK, 1, mask_code,
+                       _KV16[dtype], 1, 0, scale, 0.0)
+    rc = _native.entry("helm_decode_step")(_engine.get_engine(device), addr)
+    if rc == _native.HELM_E_UNSUPPORTED:
+        return None
+    if rc:
+        _native.check("helm_decode_step", rc)
+    return out
+
+
 def _decode_step_fast(kvcms, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                       layer_idx: int, scale: float,
                       attention_mask: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
@@ -1259,25 +1360,14 @@ def _decode_step_fast(kvcms, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     the attention kernel writes each token itself.  Returns None, having
     changed nothing, when any of that does not hold (the general path runs;
     HELM_AMD_FAST_DECODE=0 always takes it)."""
-    B, Hq, S, D = q.shape
-    kv_code = _KV16.get(q.dtype)
-    if (kv_code is None or S != 1 or D != 128 or B > _native.DECODE_MAX_SEQS
-            or not q.is_cuda or k.dtype is not q.dtype or v.dtype is not q.dtype
-            or not q.is_contiguous()):
+    if not _decode_operands_plain(q, k, v) or not _async_kv_prefetch_enabled():
         return None
-    kB, Hkv, kS, _ = k.shape
+    B, Hq, _, D = q.shape
+    kv_code = _KV16[q.dtype]
+    Hkv = k.shape[1]
     ks, vs = k.stride(), v.stride()
     kp, vp = k.data_ptr(), v.data_ptr()
     qp = q.data_ptr()
-    if (Hq > 16 * Hkv                           # more than one 16-row tile per KV head
-            or kB < B or kS != 1 or ks[3] != 1 or vs[3] != 1 or ks[1] != vs[1]
-            or (ks[1] * 2) % 16 or (kp | vp | qp | (ks[0] * 2) | (vs[0] * 2)) % 16):
-        return None
-    if (check_records_enabled() or not _async_kv_prefetch_enabled()
-            or _env_get("HELM_AMD_FAST_DECODE") == "0"
-            or _env_get("HELM_AMD_FUSED_APPEND") == "0"
-            or _env_get("HELM_AMD_KERNEL") not in (None, "", "auto", "mfma")):
-        return None
     device = q.device
     sig = (q.dtype, Hkv, D)
     layers = []
@@ -1299,22 +1389,13 @@ def _decode_step_fast(kvcms, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         layers.append(layer)
     if B > 1 and len({id(layer) for layer in layers}) != B:
         return None
-    mask_code, mbs, mhs, mptr = _native.HELM_F32, 0, 0, 0
-    m = attention_mask
-    if m is not None:
-        mask_code = _MASK_CODES.get(m.dtype)
+    margs = _NO_MASK
+    if attention_mask is not None:
         t_max = max(l._tail_tok_off + l.tail_page.used_tokens for l in layers) + 1
-        mshape = m.shape
-        if (mask_code is None or m.device != device or len(mshape) != 4
-                or mshape[0] not in (1, B) or mshape[1] not in (1, Hq) or mshape[2] != 1
-                or mshape[3] < t_max):
+        margs = _decode_mask_args(attention_mask, device, B, Hq, t_max)
+        if margs is None:
             return None
-        mst = m.stride()
-        if mst[3] != 1:
-            return None
-        mptr = m.data_ptr()
-        mbs = mst[0] if mshape[0] > 1 else 0
-        mhs = mst[1] if mshape[1] > 1 else 0
+    mptr, mbs, mhs, mask_code = margs
     # HELM's append_decode bookkeeping (kv_cache.py:145-171): the tail gains
     # the token
     _, buf, addr = _decode_args()

@@ -36,7 +36,7 @@ from helm_amd import _native
 from helm_amd.runtime import engine as _engine
 from helm_amd.runtime.kv_allocator import KVAllocator
 from helm_amd.runtime.kv_cache import (ContiguousKV, KVCacheManager, _async_kv_prefetch_enabled,
-                                       _decode_step_fast,
+                                       _decode_contiguous_fast, _decode_step_fast,
                                        _attend, _attend_device_records, _attend_layers,
                                        _attend_records, _contiguous_segments, _page_segments,
                                        _record_prefetch, perform_streaming_attention)
@@ -162,10 +162,14 @@ def _decode_batched(kvcms, q, k, v, layer_idx: int, scale: float,
 def _decode_contiguous(kvcms, q, k, v, layer_idx: int, Hkv: int, scale: float,
                        attention_mask: Optional[torch.Tensor]):
     """The contiguous fast path of a decode step (kv_offload.py:116-138):
-    every item's token written into its buffers at its position (one append
-    launch), then one attention call over the buffers' device-resident
-    virtual-page records (ContiguousKV), each item over its tokens so far
-    including this one."""
+    every item's token written into its buffers at its position and one
+    attention call over the buffers' device-resident virtual-page records
+    (ContiguousKV), each item over its tokens so far including this one; one
+    launch where the attention kernel can write the tokens, else an append
+    launch before it."""
+    out = _decode_contiguous_fast(kvcms, q, k, v, layer_idx, scale, attention_mask)
+    if out is not None:
+        return out
     for i, kvcm in enumerate(kvcms):
         kvcm._queue_contiguous(layer_idx, kvcm.cont_seq_len, k[i:i + 1], v[i:i + 1])
     _flush_appends([kvcm._appends for kvcm in kvcms])

@@ -136,3 +136,48 @@ def test_tiny_llama_with_contiguous_cache_matches_hf_greedy():
     mgr.restore()
     assert out_tokens == ref_tokens
     assert used_cont[0] and not used_cont[-1]
+
+
+@pytest.mark.parametrize("dtype,Hq,Hkv,D,layout", [
+    (torch.bfloat16, 32, 8, 128, "heads"),       # [B, 1, Hkv, D] transposed: strided heads
+    (torch.float16, 16, 1, 128, "plain"),        # a full 16-row tile
+    (torch.bfloat16, 40, 2, 128, "plain"),       # more rows than a tile: the general route
+    (torch.bfloat16, 8, 2, 128, "unaligned"),    # token rows 2 bytes off: the general route
+    (torch.bfloat16, 8, 2, 64, "plain"),         # D = 64: the general route
+    (torch.float32, 8, 2, 128, "plain"),         # fp32: the general route
+])
+@pytest.mark.parametrize("n", [1, 15, 16, 143])
+def test_contiguous_step_one_call_equals_two(dtype, Hq, Hkv, D, layout, n, monkeypatch):
+    """The step that writes the tokens in the attention launch against the
+    append launch followed by attention (HELM_AMD_FAST_DECODE=0): the same
+    bits out and in the buffers, at the first and last slots of a virtual page
+    and in the buffer's last token."""
+    B, cap = 3, 144
+    g = torch.Generator().manual_seed(n + D)
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g).to(dtype).to(DEV)
+    K, V, q = rnd(B, Hkv, n, D), rnd(B, Hkv, n, D), rnd(B, Hq, 1, D)
+    if layout == "heads":
+        kn, vn = (rnd(B, 1, Hkv, D).transpose(1, 2) for _ in range(2))
+    elif layout == "unaligned":
+        kn, vn = (rnd(B * Hkv * D + 1)[1:].view(B, Hkv, 1, D) for _ in range(2))
+    else:
+        kn, vn = rnd(B, Hkv, 1, D), rnd(B, Hkv, 1, D)
+    mask = torch.zeros(B, 1, 1, n + 1, dtype=dtype, device=DEV)
+    mask[1, ..., :n // 3] = torch.finfo(dtype).min
+    got = []
+    for fast in ("1", "0"):
+        monkeypatch.setenv("HELM_AMD_FAST_DECODE", fast)
+        mgrs = [KVCacheManager(KVAllocator(2, Hkv, D, page_size=16, dtype=dtype), 10 ** 12)
+                for _ in range(B)]
+        for b, m in enumerate(mgrs):
+            assert m.build_contiguous(2, Hkv, D, cap, DEV, dtype)
+            m._cont.arena.zero_()
+            m.prefill_contiguous(0, K[b:b + 1], V[b:b + 1])
+        out = _decode_batched(mgrs, q, kn, vn, 0, 1 / math.sqrt(D), mask)
+        got.append([out] + [m._cont.arena[0, :, :, :n + 1].clone() for m in mgrs])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    for b in range(B):
+        assert torch.equal(got[0][1 + b][0, :, n], kn[b, :, 0])
+        assert torch.equal(got[0][1 + b][1, :, n], vn[b, :, 0])
