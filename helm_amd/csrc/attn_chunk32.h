@@ -111,6 +111,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   static_assert(NW == 4 || NW == 8, "waves per workgroup");
   constexpr int SB = kChunkStage;   // 16-token blocks per stage
   constexpr bool kHiLo = chunk32_hilo(D);
+  constexpr bool kAhead = !((FEAT & kFeatMask) && D == 256);
   constexpr int NK = D / 16;        // 16-dim steps of q . k
   constexpr int NE = D / 32;        // 32-dim groups of P . V
   constexpr int CPR = D / 8;        // 16-byte chunks per token row
@@ -121,6 +122,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   constexpr bool kMask = (FEAT & kFeatMask) != 0;
   constexpr bool kCap = (FEAT & kFeatCap) != 0;
   constexpr bool kCausal = (FEAT & kFeatCausal) != 0;
+  constexpr bool kMask16 = (FEAT & kFeatMask16) != 0;
   // 16-byte-per-lane loads (1 KiB each) a wave issues per stage: a stage is
   // SB blocks of K and of V, kBlkLoads loads each, shared out over the NW
   // waves in order (wave w takes loads w * kLoads ..), all in one block per wave
@@ -195,6 +197,12 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   const int s_vis = s_row + coff;                      // row jr's last visible token
   const int s_last = (rbase + nrows - 1) / G + coff;   // the wave's last visible token
   const int s_first = rbase / G + coff;                // and its first row's
+  // causal: the workgroup's last query position; stages starting past it
+  // add nothing for any of its rows (a causal call lists a launch's pages in
+  // token order, so tokens only grow along the walk), and the walk ends
+  // there (uniform across the workgroup)
+  const int qrow_end = min(G * S, (query_block(p) + 1) * NW * kChunk32Rows);
+  const int s_last_wg = (qrow_end - 1) / G + coff;
   mf_u32x4 qop[NK];
   {
     const char* qp = reinterpret_cast<const char*>(p.q) +
@@ -233,53 +241,90 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   const int nblk = npg * bpp;
   const int nstage = (nblk + SB - 1) / SB;
 
-  // page records: window [win, win + 64) of the split's pages (the next
-  // window is read when the walk enters it, once per 64 pages)
-  typename LanesOf<Src>::type lanes = lane_pages(src, b, pg0, lane);
-  int win = 0;
-  int cur_pi = 0, cur_sub = 0;   // page (relative to pg0) and sub-block of the next view
+  // The walk's blocks, viewed 64 at a time: lane i holds block win + i of the
+  // split, its K / V addresses, valid tokens and first token offset, and ballots
+  // over the window say which blocks are partial (or empty), add nothing to any
+  // row of the wave, reach a row's causal limit, or lie past every row of the
+  // workgroup.  A stage then takes its four blocks' bits and one address by
+  // v_readlane, where walking pages and sub-blocks in scalar code took ~120
+  // scalar instructions per stage of every wave's serial path (bf16 512 tokens
+  // over 32k: 296 -> 271; D = 64, 512 over 16k: 144 -> 128 us).  The next
+  // window's records are read one window ahead.
+  struct Window {
+    uint32_t klo, khi, vlo, vhi;
+    int nt, t0;
+    uint64_t part, none, limit, end;
+  } win;
+  auto block_page = [&](int blk) -> int {
+    return min(p.bpp_log2 >= 0 ? blk >> p.bpp_log2 : blk / bpp, npg - 1);
+  };
+  // the record of the page of block w0 + lane (lane 0's position of a lane window)
+  auto load_records = [&](int w0) {
+    return lane_pages(src, b, pg0 + block_page(w0 + lane), 0);
+  };
+  typename LanesOf<Src>::type recs = load_records(0);
+  auto enter_window = [&](int w0) {
+    if (!kAhead && w0 > 0) recs = load_records(w0);
+    const int blk = w0 + lane;
+    const int pi = block_page(blk);
+    const int tok_in = (blk - pi * bpp) * kBlockTok;
+    const PageView pv = lane_own_view(src, recs, b, pg0 + pi, hk);
+    win.nt = blk < nblk ? max(0, min(pv.used - tok_in, kBlockTok)) : 0;
+    win.t0 = pv.tok_off + tok_in;
+    const uint64_t ka = reinterpret_cast<uint64_t>(pv.k) + (int64_t)tok_in * kRow;
+    const uint64_t va = reinterpret_cast<uint64_t>(pv.v) + (int64_t)tok_in * kRow;
+    win.klo = static_cast<uint32_t>(ka);
+    win.khi = static_cast<uint32_t>(ka >> 32);
+    win.vlo = static_cast<uint32_t>(va);
+    win.vhi = static_cast<uint32_t>(va >> 32);
+    win.part = __builtin_amdgcn_ballot_w64(win.nt < kBlockTok);
+    win.none = __builtin_amdgcn_ballot_w64(win.nt == 0 || (kCausal && win.t0 > s_last));
+    win.limit =
+        kCausal ? __builtin_amdgcn_ballot_w64(win.nt > 0 && win.t0 + kBlockTok - 1 > s_first) : 0;
+    // (an empty block, past the used tokens of a page shorter than the longest,
+    // says nothing: the next page's tokens may lie before its offset)
+    win.end = kCausal ? __builtin_amdgcn_ballot_w64(win.nt > 0 && win.t0 > s_last_wg) : 0;
+    if (kAhead) recs = load_records(w0 + kRecWindow);
+  };
 
-  // a stage's blocks: valid tokens and first token offset of each (kept for
-  // the stage's compute, one stage after its loads were issued), and the
-  // block this wave loads
+  // a stage's four blocks: their bits of the window's ballots, and (where a
+  // step needs them: a mask, a partial block or a causal limit) their valid
+  // tokens and first token offsets; kept for the stage's compute, one stage
+  // after its loads were issued
+  struct StageBits {
+    uint32_t part, none, limit;
+    bool end;
+  } bits[2];
   int vnt[2][SB], vt0[2][SB];
   struct OwnBlock {
     int ntok;
     const char *kb, *vb;
   };
   const int own_blk = (wave * kLoads) / (2 * kBlkLoads);
-  // (a stage never straddles two record windows: window w starts at block
-  // 64 w bpp of the split, a multiple of the stage's SB = 4 blocks, so the
-  // window is entered at a stage's first block; blocks past the split's end
-  // have no tokens and their views are never dereferenced)
-  static_assert(kRecWindow % SB == 0, "record windows start at stage boundaries");
-  auto view_stage = [&](int st, int (&ntok)[SB], int (&tok0)[SB], OwnBlock& ob) {
-    if (cur_pi - win >= kRecWindow) {   // uniform: the stage lies in the next window
-      win += kRecWindow;
-      lanes = lane_pages(src, b, pg0 + win, lane);
-    }
-    int own_pi = cur_pi, own_tok_in = 0;
+  static_assert(kRecWindow % SB == 0, "windows start at stage boundaries");
+  auto view_stage = [&](int st, StageBits& sb, int (&ntok)[SB], int (&tok0)[SB], OwnBlock& ob) {
+    const int at = (st * SB) % kRecWindow;
+    if (at == 0) enter_window(st * SB);   // uniform
+    constexpr uint32_t kAll = (1u << SB) - 1;
+    sb.part = static_cast<uint32_t>(win.part >> at) & kAll;
+    sb.none = static_cast<uint32_t>(win.none >> at) & kAll;
+    sb.limit = static_cast<uint32_t>(win.limit >> at) & kAll;
+    sb.end = (win.end >> at) & 1;
+    if (kMask || (sb.part | sb.limit)) {
 #pragma unroll
-    for (int j = 0; j < SB; ++j) {
-      const PageMeta pm = lane_page_meta(src, lanes, b, pg0 + cur_pi, cur_pi - win);
-      const int tok_in = cur_sub * kBlockTok;
-      const int nt = st * SB + j < nblk ? sclamp(pm.used - tok_in, 0, kBlockTok) : 0;
-      ntok[j] = nt;
-      tok0[j] = pm.tok_off + tok_in;
-      if (j == own_blk) {
-        ob.ntok = nt;
-        own_pi = cur_pi;
-        own_tok_in = tok_in;
-      }
-      if (++cur_sub == bpp) {
-        cur_sub = 0;
-        ++cur_pi;
+      for (int j = 0; j < SB; ++j) {
+        ntok[j] = __builtin_amdgcn_readlane(win.nt, at + j);
+        tok0[j] = __builtin_amdgcn_readlane(win.t0, at + j);
       }
     }
-    // the addresses of the one block this wave loads
-    const PageView pv = lane_page_view(src, lanes, b, pg0 + own_pi, own_pi - win, hk);
-    ob.kb = pv.k + own_tok_in * kRow;
-    ob.vb = pv.v + own_tok_in * kRow;
+    const int own = at + own_blk;
+    ob.ntok = __builtin_amdgcn_readlane(win.nt, own);
+    ob.kb = reinterpret_cast<const char*>(
+        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(win.khi, own) << 32) |
+        (uint32_t)__builtin_amdgcn_readlane(win.klo, own));
+    ob.vb = reinterpret_cast<const char*>(
+        ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(win.vhi, own) << 32) |
+        (uint32_t)__builtin_amdgcn_readlane(win.vlo, own));
   };
 
   // this wave's loads of a stage straight from memory into LDS (no VGPRs):
@@ -318,58 +363,62 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
            8 * (nl & 1);
   };
 
-  // additive mask of row jr for the step of blocks bp, bp + 1 of a stage:
-  // tokens 8hh .. 8hh + 7 of each block, bounded by its valid tokens, as
-  // loaded: words 0 .. 7 of a block for an fp32 mask, 0 .. 3 (two tokens each)
-  // for a 16-bit one.  A whole block's tokens are 16-byte loads at the mask's
-  // own alignment; a partial block's go one by one, the index clamped to its
-  // last valid token.  Element loads of every block, 16 per step, had bound the
-  // masked chunk, and a zero mask was added all the same: bf16 512 over 8,192
-  // tokens under a 4,096-token window, 32 / 8 heads, 187 -> 121 us; D = 256, 512
-  // over 4,700, soft-capped, 203 -> 106 us (tanhf per score was the rest).
-  // (Whole-vector values: element stores from several branches would put the
-  // words in scratch memory.)
-  mf_u32x8 mk_next[2];
-  auto load_block_mask = [&](int nt, int tok0) -> mf_u32x8 {
+  // additive mask of row jr for a stage's blocks: tokens 8hh .. 8hh + 7 of
+  // each, bounded by its valid tokens, as loaded: eight words for an fp32 mask,
+  // four (two tokens each) for a 16-bit one.  A whole block's tokens are 16-byte
+  // loads at the mask's own alignment; a partial block's go one by one, the index
+  // clamped to its last valid token.  A stage's masks are loaded with its K / V, one
+  // stage ahead, or, where the registers for two stages' are not there (fp32
+  // masks; D = 128 soft-capped), at the stage's start before the next stage's
+  // K / V: a load after those would have to wait for them too.  Element loads of every step, converted and added
+  // even where zero, had bound the masked chunk (bf16 512 over 8,192 tokens under
+  // a 4,096-token window, 32 / 8 heads: 187 us, now 108; D = 256, 512 over 4,700,
+  // soft-capped: 203, now 99).
+  typedef typename std::conditional<kMask16, mf_u32x4, mf_u32x8>::type MaskWords;
+  constexpr bool kMaskAhead = kMask16 && !(kCap && D == 128);
+  MaskWords mkw[kMaskAhead ? 2 : 1][SB];
+  auto load_block_mask = [&](int nt, int tok0) -> MaskWords {
     const MaskRow mb = mrow + tok0;
     if (__builtin_expect(nt == kBlockTok, 1)) {
       const char* src = (mb + 8 * hh).base;
       const mf_u32x4 a = load16_any(src);
-      const mf_u32x4 c = p.mask_dt == HELM_F32 ? load16_any(src + 16) : mf_u32x4{0u, 0u, 0u, 0u};
-      return mf_u32x8{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+      if constexpr (kMask16) {
+        return a;
+      } else {
+        const mf_u32x4 c = load16_any(src + 16);
+        return mf_u32x8{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+      }
     }
-    if (nt == 0) return mf_u32x8{0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-    auto f32 = [&](int i) -> uint32_t {
-      return mb.template bits<false>(min(8 * hh + i, nt - 1));
+    if (nt == 0) return MaskWords(0u);
+    auto at = [&](int i) -> uint32_t {
+      return mb.template bits<kMask16>(min(8 * hh + i, nt - 1));
     };
-    auto h16 = [&](int i) -> uint32_t {
-      return mb.template bits<true>(min(8 * hh + i, nt - 1)) |
-             (uint32_t)mb.template bits<true>(min(8 * hh + i + 1, nt - 1)) << 16;
-    };
-    if (p.mask_dt == HELM_F32)
-      return mf_u32x8{f32(0), f32(1), f32(2), f32(3), f32(4), f32(5), f32(6), f32(7)};
-    return mf_u32x8{h16(0), h16(2), h16(4), h16(6), 0u, 0u, 0u, 0u};
+    if constexpr (kMask16)
+      return mf_u32x4{at(0) | at(1) << 16, at(2) | at(3) << 16, at(4) | at(5) << 16,
+                      at(6) | at(7) << 16};
+    else
+      return mf_u32x8{at(0), at(1), at(2), at(3), at(4), at(5), at(6), at(7)};
   };
-  auto load_step_mask = [&](const int (&ntok)[SB], const int (&tok0)[SB], int bp) {
+  auto load_stage_mask = [&](const int (&ntok)[SB], const int (&tok0)[SB], MaskWords (&w)[SB]) {
     if constexpr (kMask) {
-      mk_next[0] = load_block_mask(ntok[bp], tok0[bp]);
-      mk_next[1] = load_block_mask(ntok[bp + 1], tok0[bp + 1]);
+#pragma unroll
+      for (int j = 0; j < SB; ++j) w[j] = load_block_mask(ntok[j], tok0[j]);
     }
   };
-  // any bit of the step's mask words set (a zero mask adds nothing to any score)
-  auto mask_bits = [&](const mf_u32x8& a, const mf_u32x8& b) -> uint32_t {
-    const mf_u32x8 w = a | b;   // (a 16-bit mask's last four words are zero)
-    return w[0] | w[1] | w[2] | w[3] | w[4] | w[5] | w[6] | w[7];
+  // any bit of the mask words set (a zero mask adds nothing to any score)
+  auto mask_bits = [&](const MaskWords& w) -> uint32_t {
+    uint32_t any = w[0] | w[1] | w[2] | w[3];
+    if constexpr (!kMask16) any |= w[4] | w[5] | w[6] | w[7];
+    return any;
   };
   // a block's eight mask values in fp32
-  auto mask_values = [&](const mf_u32x8& w, float* mk) {
-    if (p.mask_dt == HELM_F32) {
+  auto mask_values = [&](const MaskWords& w, float* mk) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) mk[i] = __uint_as_float(w[i]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (kMask16)
         mk[i] = mrow.template widen<true>((i & 1) ? w[i >> 1] >> 16 : w[i >> 1] & 0xffffu);
+      else
+        mk[i] = __uint_as_float(w[i]);
     }
   };
 
@@ -377,17 +426,11 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   {
     OwnBlock ob;
     if (nstage > 0) {
-      view_stage(0, vnt[0], vt0[0], ob);
+      view_stage(0, bits[0], vnt[0], vt0[0], ob);
       dma_stage(ob, lds0);
-      if (wave_rows) load_step_mask(vnt[0], vt0[0], 0);
+      if (kMaskAhead && wave_rows) load_stage_mask(vnt[0], vt0[0], mkw[0]);
     }
   }
-  // causal: the workgroup's last query position; stages starting past it
-  // add nothing for any of its rows (a causal call lists a launch's pages in
-  // token order, so tokens only grow along the walk), and the walk ends
-  // there (uniform across the workgroup)
-  const int qrow_end = min(G * S, (query_block(p) + 1) * NW * kChunk32Rows);
-  const int s_last_wg = (qrow_end - 1) / G + coff;
   bool done = false;
   // stage st (view slot K = st % 2) computes from `cur` while the loads of
   // stage st + 1 go into `nxt` (the buffer stage st - 1 computed from)
@@ -396,9 +439,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
     const int (&ntok_c)[SB] = vnt[K];
     const int (&tok0_c)[SB] = vt0[K];
     if constexpr (kCausal) {
-      // (an empty block, past the used tokens of a page shorter than the
-      // longest, says nothing: the next page's tokens may lie before its offset)
-      if (ntok_c[0] > 0 && tok0_c[0] > s_last_wg) {
+      if (bits[K].end) {
         __builtin_amdgcn_s_waitcnt(0x0F70);   // this stage's loads land before the exit
         done = true;
         return;
@@ -408,10 +449,13 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
     // wave is done with the other buffer, which the next stage's loads fill
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
     __syncthreads();
+    if (!kMaskAhead && wave_rows) load_stage_mask(ntok_c, tok0_c, mkw[0]);
     if (st + 1 < nstage) {
       OwnBlock ob;
-      view_stage(st + 1, vnt[K ^ 1], vt0[K ^ 1], ob);
+      view_stage(st + 1, bits[K ^ 1], vnt[K ^ 1], vt0[K ^ 1], ob);
       dma_stage(ob, nxt);
+      if constexpr (kMaskAhead)
+        if (wave_rows) load_stage_mask(vnt[K ^ 1], vt0[K ^ 1], mkw[K ^ 1]);
     }
     if (wave_rows) {
       // q . k of the step of blocks bp, bp + 1: S^T for the wave's 32 rows
@@ -437,17 +481,9 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
       // (uniform tests): both blocks empty (an empty block holds zeros and
       // -inf logits), or, causal, every token past the wave's last query
       // position
-      auto idle_step = [&](int bp) -> bool {
-        const int nt0 = ntok_c[bp], nt1 = ntok_c[bp + 1];
-        if (nt0 == 0 && nt1 == 0) return true;
-        if constexpr (kCausal)
-          return (nt0 == 0 || tok0_c[bp] > s_last) &&
-                 (nt1 == 0 || tok0_c[bp + 1] > s_last);
-        return false;
-      };
+      auto idle_step = [&](int bp) -> bool { return ((bits[K].none >> bp) & 3) == 3; };
       // logits, online softmax and P . V of one step
       auto finish = [&](int bp, const mf_f32x16& sc, bool add_mask, const float (&mk)[16]) {
-        const int nt0 = ntok_c[bp], nt1 = ntok_c[bp + 1];
         float x[16];
         if constexpr (kCap) {
 #pragma unroll
@@ -468,13 +504,14 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
         // the causal limit when a block's last token is past the wave's first
         // query position, the valid-token limit when a block is partial
         if constexpr (kCausal) {
-          if (__builtin_expect(max(tok0_c[bp], tok0_c[bp + 1]) + kBlockTok - 1 > s_first, 0)) {
+          if (__builtin_expect((bits[K].limit >> bp) & 3, 0)) {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
               if (tok0_c[bp + (r >> 3)] + 8 * hh + (r & 7) > s_vis) x[r] = -INFINITY;
           }
         }
-        if (__builtin_expect(nt0 < kBlockTok || nt1 < kBlockTok, 0)) {
+        if (__builtin_expect((bits[K].part >> bp) & 3, 0)) {
+          const int nt0 = ntok_c[bp], nt1 = ntok_c[bp + 1];
 #pragma unroll
           for (int r = 0; r < 16; ++r)
             if (8 * hh + (r & 7) >= ((r >> 3) ? nt1 : nt0)) x[r] = -INFINITY;
@@ -533,16 +570,6 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
       {
 #pragma unroll
         for (int bp = 0; bp < SB; bp += 2) {     // the step's blocks bp, bp + 1
-          // the mask of the next step is loaded now, one step ahead of its use
-          mf_u32x8 mw0, mw1;
-          if constexpr (kMask) {
-            mw0 = mk_next[0];
-            mw1 = mk_next[1];
-            if (bp + 2 < SB)
-              load_step_mask(ntok_c, tok0_c, bp + 2);
-            else if (st + 1 < nstage)
-              load_step_mask(vnt[K ^ 1], vt0[K ^ 1], 0);
-          }
           if (__builtin_expect(idle_step(bp), 0)) continue;
           // masked, a step whose every mask value is <= -1e30 while every
           // row's max is already above -1e20 adds exactly nothing (each
@@ -550,10 +577,11 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
           float mk[16];
           bool add_mask = false;
           if constexpr (kMask) {
-            add_mask = __builtin_amdgcn_ballot_w64(mask_bits(mw0, mw1) != 0u) != 0;
+            const MaskWords &w0 = mkw[kMaskAhead ? K : 0][bp], &w1 = mkw[kMaskAhead ? K : 0][bp + 1];
+            add_mask = __builtin_amdgcn_ballot_w64(mask_bits(w0 | w1) != 0u) != 0;
             if (add_mask) {
-              mask_values(mw0, mk);
-              mask_values(mw1, mk + 8);
+              mask_values(w0, mk);
+              mask_values(w1, mk + 8);
               float mm = mk[0];
 #pragma unroll
               for (int r = 1; r < 16; ++r) mm = fmaxf(mm, mk[r]);

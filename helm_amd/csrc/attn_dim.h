@@ -14,10 +14,8 @@ namespace {
 
 template <typename T, class Src, int FEAT, int D>
 hipError_t launch_dim_feat(const LaunchSpec& s, const Src& src, hipStream_t st) {
-  // the chunk kernels read a mask's element type at run time
-  constexpr int CF = FEAT & ~kFeatMask16;
   if (s.p.row_waves && s.nw == 4)
-    HELM_ATTN_LAUNCH((chunk32_mfma_dim_kernel<T, Src, CF, 4, D>), s.grid, dim3(256), s.p, src);
+    HELM_ATTN_LAUNCH((chunk32_mfma_dim_kernel<T, Src, FEAT, 4, D>), s.grid, dim3(256), s.p, src);
   else if (!s.p.row_waves && s.nw == 4)
     HELM_ATTN_LAUNCH((decode_mfma_dim_kernel<T, Src, FEAT, D>), s.grid, dim3(256), s.p, src);
   else

@@ -40,13 +40,13 @@ hipError_t launch_generic(const LaunchSpec& s, hipStream_t st) {
 // Matrix-core kernels: D = 128, q and KV of the same 16-bit type.
 template <typename T, class Src, int FEAT>
 hipError_t launch_mfma_feat(const LaunchSpec& s, const Src& src, hipStream_t st) {
-  // the chunk kernels read a mask's element type at run time
+  // the 16-row chunk kernel reads a mask's element type at run time
   constexpr int CF = FEAT & ~kFeatMask16;
   if (s.p.row_waves == 2) {
     if (s.nw == 8)
-      HELM_ATTN_LAUNCH((chunk32_mfma_kernel<T, Src, CF, 8>), s.grid, dim3(512), s.p, src);
+      HELM_ATTN_LAUNCH((chunk32_mfma_kernel<T, Src, FEAT, 8>), s.grid, dim3(512), s.p, src);
     else
-      HELM_ATTN_LAUNCH((chunk32_mfma_kernel<T, Src, CF, 4>), s.grid, dim3(256), s.p, src);
+      HELM_ATTN_LAUNCH((chunk32_mfma_kernel<T, Src, FEAT, 4>), s.grid, dim3(256), s.p, src);
   } else if (s.p.row_waves)
     HELM_ATTN_LAUNCH((chunk_mfma_kernel<T, Src, CF>), s.grid, dim3(256), s.p, src);
   else if (s.nw == 8)

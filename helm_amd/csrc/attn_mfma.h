@@ -59,8 +59,8 @@ constexpr float kMfmaSlack = 8.f;
 // D = 64's blocks are 4 KiB of K/V: twice as many are in flight per wave.
 constexpr int mfma_bufs(int D) { return D == 64 ? 4 : HELM_MFMA_NBUF; }
 
-// kFeatMask16: the mask is 16-bit (bf16 / fp16); only the decode kernel
-// reads it at that width (the chunk kernels read the element type at run time)
+// kFeatMask16: the mask is 16-bit (bf16 / fp16); the decode and 32-row chunk
+// kernels read it at that width (the 16-row chunk kernel at run time)
 enum MfmaFeat { kFeatMask = 1, kFeatCap = 2, kFeatCausal = 4, kFeatMask16 = 8 };
 
 typedef __bf16 mf_bf16x8 __attribute__((ext_vector_type(8)));
@@ -163,29 +163,27 @@ __device__ __forceinline__ mf_u32x4 load16_any(const char* p) {
 // the N scores of a lane.  Logits far below the cap (|x k| <= 2^-2.5 for every
 // score of the wave, |logit| <= 8.8 at a cap of 50: the usual case) take the
 // odd Taylor polynomial of tanh through y^7, whose first left-out term is below
-// 2.1e-8 of the result there, an eighth of an fp32 ulp; up to |x k| <= 1/2 the
-// one through y^13 (8.9e-8); any other step tanhf.
+// 2.1e-8 of the result there, a third of an fp32 half ulp; k and cap sit in its
+// coefficients (x times a polynomial in x^2: five instructions a score), which
+// holds while their powers stay in fp32's range: |k| in [2^-20, 2^8], far around
+// every head dim and cap in use.  Any other step takes tanhf (for every step it
+// had cost as much as the softmax: bf16 chunk of 512 over 8,192, 32 / 8 heads,
+// 4,096-token window, capped: 236 us, now 134).
 template <int N>
 __device__ __forceinline__ void softcap_scores(float (&x)[N], float k, float cap) {
   float top = fabsf(x[0]);
 #pragma unroll
   for (int r = 1; r < N; ++r) top = fmaxf(top, fabsf(x[r]));
-  top *= k;
-  constexpr float c1 = -1.f / 3.f, c2 = 2.f / 15.f, c3 = -17.f / 315.f, c4 = 62.f / 2835.f,
-                  c5 = -1382.f / 155925.f, c6 = 21844.f / 6081075.f;
-  const float kc = k * cap;
-  if (__builtin_expect(!__builtin_amdgcn_ballot_w64(!(top <= 0.1767767f)), 1)) {
+  const float ak = fabsf(k);
+  const bool in_range = ak >= 0x1p-20f && ak <= 0x1p8f;
+  if (__builtin_expect(in_range && !__builtin_amdgcn_ballot_w64(!(top * ak <= 0.1767767f)), 1)) {
+    const float kk = k * k, a0 = k * cap;
+    const float a1 = a0 * kk * (-1.f / 3.f), a2 = a0 * kk * kk * (2.f / 15.f);
+    const float a3 = a0 * kk * kk * kk * (-17.f / 315.f);
 #pragma unroll
     for (int r = 0; r < N; ++r) {
-      const float y = x[r] * k, z = y * y;
-      x[r] = x[r] * kc * fmaf(z, fmaf(z, fmaf(z, c3, c2), c1), 1.f);
-    }
-  } else if (!__builtin_amdgcn_ballot_w64(!(top <= 0.5f))) {
-#pragma unroll
-    for (int r = 0; r < N; ++r) {
-      const float y = x[r] * k, z = y * y;
-      const float h = fmaf(z, fmaf(z, fmaf(z, c6, c5), c4), c3);
-      x[r] = x[r] * kc * fmaf(z, fmaf(z, fmaf(z, h, c2), c1), 1.f);
+      const float z = x[r] * x[r];
+      x[r] *= fmaf(z, fmaf(z, fmaf(z, a3, a2), a1), a0);
     }
   } else {
 #pragma unroll
@@ -280,26 +278,29 @@ __device__ __forceinline__ PageView lane_page_view(const DescSrc& s, const DescL
   return pv;
 }
 
-// Used tokens and token offset of page i of the split (uniform), without its
-// addresses: what a walk needs for the blocks it does not load itself.
-struct PageMeta {
-  int used;
-  int tok_off;
-};
-__device__ __forceinline__ PageMeta lane_page_meta(const PoolSrc& s, const PoolLanes&, int b,
-                                                   int pg, int) {
-  const int T = sload(s.seq_lens + b);
-  PageMeta pm;
-  pm.tok_off = pg * s.page_size;
-  pm.used = min(s.page_size, T - pm.tok_off);
-  return pm;
+// The page `pg` (per lane) whose record this lane holds: head-hk K / V bases,
+// used tokens, token offset.
+__device__ __forceinline__ PageView lane_own_view(const PoolSrc& s, const PoolLanes& L, int b,
+                                                  int pg, int hk) {
+  PageView pv;
+  const int64_t off = (int64_t)L.slot * s.slot_stride_b + hk * s.head_stride_b;
+  pv.k = s.k_pool + off;
+  pv.v = s.v_pool + off;
+  pv.tok_off = pg * s.page_size;
+  pv.used = min(s.page_size, sload(s.seq_lens + b) - pv.tok_off);
+  pv.head_stride_b = 0;
+  return pv;
 }
-__device__ __forceinline__ PageMeta lane_page_meta(const DescSrc&, const DescLanes& L, int, int,
-                                                   int i) {
-  PageMeta pm;
-  pm.used = __builtin_amdgcn_readlane(L.used, i);
-  pm.tok_off = __builtin_amdgcn_readlane(L.tok_off, i);
-  return pm;
+__device__ __forceinline__ PageView lane_own_view(const DescSrc& s, const DescLanes& L, int, int,
+                                                  int hk) {
+  const uint64_t off = (uint64_t)(uint32_t)L.head_stride * (uint32_t)(hk * s.elem_bytes);
+  PageView pv;
+  pv.k = reinterpret_cast<const char*>((((uint64_t)L.khi << 32) | L.klo) + off);
+  pv.v = reinterpret_cast<const char*>((((uint64_t)L.vhi << 32) | L.vlo) + off);
+  pv.used = L.used;
+  pv.tok_off = L.tok_off;
+  pv.head_stride_b = 0;
+  return pv;
 }
 
 // One 16-token block of the online-softmax recurrence on the matrix cores:

@@ -40,8 +40,9 @@ def _mask(kind, S, T, dtype):
     pos = torch.arange(T - S, T)[:, None]
     key = torch.arange(T)[None, :]
     seen = key <= pos
-    if kind == "window":
+    if kind.startswith("window"):
         seen = seen & (key > pos - max(1, T // 3))
+    dtype = torch.float32 if kind == "window_f32" else dtype
     low = torch.finfo(dtype).min
     m = torch.zeros(S, T, dtype=dtype).masked_fill_(~seen, low)
     if kind == "first_row_masked":      # one row with no visible key: equal weights
@@ -61,7 +62,10 @@ def _mask(kind, S, T, dtype):
     (4, 1, 150, [16] * 68 + [7]),        # several workgroups, past one record window
 ])
 @pytest.mark.parametrize("kind,cap", [("none", None), ("causal", None), ("window", None),
-                                      ("window", 5.0), ("first_row_masked", None)])
+                                      ("window", 5.0),      # logits near the cap: tanhf
+                                      ("window", 50.0),     # far below it: the polynomial
+                                      ("window_f32", None), ("window_f32", 50.0),
+                                      ("first_row_masked", None)])
 def test_streaming_matches_fp64(D, dtype, Hq, Hkv, S, sizes, kind, cap):
     T = sum(sizes)
     if kind == "causal" and S == 1 or kind == "none" and S > 1 or T < S and kind != "causal":
