@@ -314,8 +314,10 @@ int chunk_pps(const Plan& pl, int D, double units, double rows, double pages, do
   const double cus = device_cus();
   int best_pps = (int)std::ceil(P);
   double best = -1.0;
-  for (int s = 1; s <= 64 && s <= P; ++s) {
+  for (int s = 1; s <= 64; ++s) {
     const int pps = (int)std::ceil(P / s);
+    // (the workspace query counts on no automatic split being shorter)
+    if (s > 1 && pps < min_pps(pl.bpp, kWaves)) break;
     const double n = std::ceil(P / pps);
     const double stages = pps * (double)pl.bpp / kChunkStage;
     const double share = walk > 0.75 ? std::ceil(units * n / cus) : units * n * walk / cus;
@@ -1221,6 +1223,16 @@ int helm_paged_decode_attn(const void* q, void* out, const void* k_pool,
                                  min_pps(pl.bpp, pl.nw), max_pps_of(pl));
       if ((max_pages + cand - 1) / cand <= max_splits_of(pl)) pl.pps = cand;
     }
+    pl.max_splits = std::max(1, (max_pages + pl.pps - 1) / pl.pps);
+    pl.fused = fused_merge(pl.max_splits);
+    size_plan(pl, B, Hkv, D);
+    settle_fused(pl, B, Hkv);
+  }
+  // a workspace below a query chunk's estimated split count: fewer splits, down
+  // to the single one that needs no partials
+  while (ws_bytes < pl.total() && pl.row_waves == 2 && pages_per_split <= 0 &&
+         env_int("HELM_AMD_PPS", 0) <= 0 && pl.max_splits > 1) {
+    pl.pps = (max_pages + pl.max_splits - 2) / (pl.max_splits - 1);
     pl.max_splits = std::max(1, (max_pages + pl.pps - 1) / pl.pps);
     pl.fused = fused_merge(pl.max_splits);
     size_plan(pl, B, Hkv, D);

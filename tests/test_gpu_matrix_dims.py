@@ -123,3 +123,19 @@ def test_first_prompt_block_order(D, Hq, Hkv, S, monkeypatch):
         torch.arange(S)[None, :] > torch.arange(S)[:, None], -math.inf)
     ref = A.attention_fp64_batched(q[0], K[0], V[0], mask=causal)
     assert (out[0].double().cpu() - ref).abs().max().item() <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_pool_chunk_of_few_rows_fits_the_queried_workspace(D):
+    """34 query rows per KV head over a long context: the split estimate wants
+    as many splits as it may have, and the workspace query covers them."""
+    w = W.Workload("rows", 1, 4, 2, D, torch.bfloat16, T=5000, page_size=16)
+    case = W.make_pool_case(w, seed=D, device=DEV)
+    g = torch.Generator().manual_seed(D)
+    q = (1.5 * torch.randn(1, 4, 17, D, generator=g)).to(torch.bfloat16)
+    out = paged_decode_attention(q.to(DEV), case["k_pool"], case["v_pool"], case["table"],
+                                 case["lens"], max_pages=case["max_pages"])
+    rows = case["pool"][case["table"][0].long()].cpu()
+    kv = rows.permute(1, 2, 0, 3, 4).reshape(2, 2, -1, D)[:, :, :5000]
+    ref = A.attention_fp64_batched(q[0], kv[0], kv[1])
+    assert (out[0].double().cpu() - ref).abs().max().item() <= TOL[torch.bfloat16]
