@@ -56,8 +56,10 @@ constexpr float kMfmaSlack = 8.f;
 #ifndef HELM_MFMA_NBUF
 #define HELM_MFMA_NBUF 2
 #endif
-// D = 64's blocks are 4 KiB of K/V: twice as many are in flight per wave.
-constexpr int mfma_bufs(int D) { return D == 64 ? 4 : HELM_MFMA_NBUF; }
+// D = 64's blocks are half as large: two in flight (f16, four sequences of
+// 3k-16k tokens, 32 / 8 heads: 2 buffers 18.0 us, 3 17.3, 4 17.5, 6 17.9; one of
+// 700, 12 heads: 7.2, 7.1, 7.3, 7.7).
+constexpr int mfma_bufs(int D) { return D == 64 ? 3 : HELM_MFMA_NBUF; }
 
 // kFeatMask16: the mask is 16-bit (bf16 / fp16); the decode and 32-row chunk
 // kernels read it at that width (the 16-row chunk kernel at run time)
@@ -125,9 +127,15 @@ template <> struct MfmaOps<f16_t> {
     typedef float f2 __attribute__((ext_vector_type(2)));
     const h2 h = __builtin_convertvector((f2){w0, w1}, h2);
     hi = __builtin_bit_cast(uint32_t, h);
-    const f2 back = __builtin_convertvector(h, f2);
-    lo = __builtin_bit_cast(uint32_t,
-                            __builtin_convertvector((f2){w0 - back[0], w1 - back[1]}, h2));
+    // w - hi, exact: v_fma_mix_f32 reads the f16 half in place (the compiler
+    // would convert each half to fp32 first, one more instruction per weight;
+    // D = 64 chunk of 777 over 2,777, 14 / 2 heads: 30.1 -> 29.2 us)
+    f2 r;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r[0]) : "v"(hi), "v"(w0));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+        : "=v"(r[1])
+        : "v"(hi), "v"(w1));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, h2));
   }
 };
 
