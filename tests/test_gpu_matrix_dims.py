@@ -139,3 +139,33 @@ def test_pool_chunk_of_few_rows_fits_the_queried_workspace(D):
     kv = rows.permute(1, 2, 0, 3, 4).reshape(2, 2, -1, D)[:, :, :5000]
     ref = A.attention_fp64_batched(q[0], kv[0], kv[1])
     assert (out[0].double().cpu() - ref).abs().max().item() <= TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("D,S", [(64, 1), (256, 1), (64, 40), (128, 40), (256, 40)])
+def test_pool_call_with_smaller_workspaces(D, S):
+    """Ever smaller workspaces: fewer splits (chunks) or the element-wise
+    kernel's plan (D = 64, 256), the same result, until the call is refused;
+    a decode call is served down to what the element-wise plan needs."""
+    from helm_amd import _native, paged
+    w = W.Workload("ws", 1, 10, 2, D, torch.bfloat16, T=1500, page_size=16)
+    case = W.make_pool_case(w, seed=D + S, device=DEV)
+    g = torch.Generator().manual_seed(D + S)
+    q = (1.5 * torch.randn(1, 10, S, D, generator=g)).to(torch.bfloat16)
+    args, keep = paged._decode_args(q.to(DEV), case["k_pool"], case["v_pool"], case["table"],
+                                    case["lens"], case["max_pages"], 0, None, None, None, None, 0)
+    rows = case["pool"][case["table"][0].long()].cpu()
+    kv = rows.permute(1, 2, 0, 3, 4).reshape(2, 2, -1, D)[:, :, :1500]
+    ref = A.attention_fp64_batched(q[0], kv[0], kv[1])
+    size, served = args[-2], 0
+    while size > (64 << 10):
+        args[-2] = size
+        keep["out"].zero_()
+        try:
+            _native.call("helm_paged_decode_attn", *args)
+        except ValueError as e:
+            assert "workspace" in str(e)
+            break
+        assert (keep["out"][0].double().cpu() - ref).abs().max().item() <= TOL[torch.bfloat16]
+        served += 1
+        size = size * 3 // 4
+    assert served >= 2
