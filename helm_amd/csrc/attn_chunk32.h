@@ -26,8 +26,10 @@
 //           exactly the weights P . V used (packed dot products with ones), so
 //           that each output row is an exact weighted mean of V under the
 //           rounded weights (their rounding perturbs the weights by <= 2^-9
-//           relative, bf16, and the mean by that times the spread of V).  HELM_CHUNK32_HILO=1 builds the split into hi and lo
-//           16-bit parts instead (weights to ~2^-17, one more MFMA per group).
+//           relative, bf16, and the mean by that times the spread of V).
+//           (D = 128; HELM_CHUNK32_HILO=1 builds hi + lo there, weights to
+//           ~2^-17, one more MFMA per group.  At D = 64 and 256 the weights
+//           enter in weight_parts parts, one MFMA per part and group.)
 // Online softmax per query row with the lazy rescale of the decode kernel, in
 // base-2 units (logits scaled by log2(e) with the softmax scale, weights
 // 2^(x - m); the partials' max goes out in natural units).
@@ -69,14 +71,17 @@ template <int D>
 __device__ __forceinline__ int swz(int t) {
   return D == 64 ? ((t & 2) << 1) | (t >> 2) : ((t & 3) << 2) | (t >> 2);
 }
-// P . V with the weights split into 16-bit hi and lo parts or, at D = 128,
-// rounded once to 16 bits (a query chunk is bound by the matrix cores, and the
-// single rounding stays far inside the tolerance; HELM_CHUNK32_HILO=1 builds
-// the split there too)
+// P . V with the weights in 16-bit parts (weight_parts) or, at D = 128, rounded
+// once to 16 bits (a query chunk is bound by the matrix cores, and the single
+// rounding stays far inside the tolerance; HELM_CHUNK32_HILO=1 builds hi + lo
+// there too)
 #ifndef HELM_CHUNK32_HILO
 #define HELM_CHUNK32_HILO 0
 #endif
-constexpr bool chunk32_hilo(int D) { return D != 128 || HELM_CHUNK32_HILO; }
+template <typename T>
+constexpr int chunk32_parts(int D) {
+  return D != 128 ? weight_parts<T>(D) : HELM_CHUNK32_HILO ? 2 : 1;
+}
 constexpr float kLog2E = 1.4426950408889634f;   // log2(e)
 constexpr float kLn2 = 0.6931471805599453f;     // ln(2)
 
@@ -110,7 +115,7 @@ template <typename T, class Src, int FEAT, int NW, int D>
 __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src& src) {
   static_assert(NW == 4 || NW == 8, "waves per workgroup");
   constexpr int SB = kChunkStage;   // 16-token blocks per stage
-  constexpr bool kHiLo = chunk32_hilo(D);
+  constexpr int kParts = chunk32_parts<T>(D);
   constexpr bool kAhead = !((FEAT & kFeatMask) && D == 256);
   constexpr int NK = D / 16;        // 16-dim steps of q . k
   constexpr int NE = D / 32;        // 32-dim groups of P . V
@@ -226,7 +231,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
 
   float m = -INFINITY;   // running max of row jr (same in both halves)
   // this lane's share of row jr's weight sum: of the fp32 weights where P . V
-  // takes them as hi + lo, else of exactly the rounded weights it takes (packed
+  // takes them in parts, else of exactly the rounded weights it takes (packed
   // dot products with ones: half the matrix-core time that a ones column of
   // P . V takes, and no accumulator tile; bf16 512 tokens over 32k, 32 / 8 heads:
   // 303 -> 299 us)
@@ -536,23 +541,26 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
             }
         }
         const float base = (m == -INFINITY) ? 0.f : m;
-        uint32_t hw[8], lw[8];
+        uint32_t hw[8], lw[8], ew[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           const float w0 = sexp(x[2 * q] - base), w1 = sexp(x[2 * q + 1] - base);
-          if constexpr (kHiLo) {
+          if constexpr (kParts == 3) {
+            lsum += w0 + w1;
+            Ops::split3(w0, w1, hw[q], lw[q], ew[q]);
+          } else if constexpr (kParts == 2) {
             lsum += w0 + w1;
             Ops::split2(w0, w1, hw[q], lw[q]);
           } else {
             hw[q] = Ops::pk(w0, w1);
-            lw[q] = 0u;
             lsum = dot2<T>(hw[q], Ops::ones8()[0], lsum);
           }
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const mf_u32x4 phi = mf_u32x4{hw[4 * u], hw[4 * u + 1], hw[4 * u + 2], hw[4 * u + 3]};
-          const mf_u32x4 plo = mf_u32x4{lw[4 * u], lw[4 * u + 1], lw[4 * u + 2], lw[4 * u + 3]};
+          auto pop = [&](const uint32_t (&w)[8]) {
+            return mf_u32x4{w[4 * u], w[4 * u + 1], w[4 * u + 2], w[4 * u + 3]};
+          };
           mf_u32x4 vop[NE];
 #pragma unroll
           for (int e = 0; e < NE; ++e) {
@@ -561,10 +569,13 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
             vop[e] = mf_u32x4{a0.x, a0.y, a1.x, a1.y};
           }
 #pragma unroll
-          for (int e = 0; e < NE; ++e) o[e] = M32::mma(phi, vop[e], o[e]);
-          if constexpr (kHiLo)
+          for (int e = 0; e < NE; ++e) o[e] = M32::mma(pop(hw), vop[e], o[e]);
+          if constexpr (kParts >= 2)
 #pragma unroll
-            for (int e = 0; e < NE; ++e) o[e] = M32::mma(plo, vop[e], o[e]);
+            for (int e = 0; e < NE; ++e) o[e] = M32::mma(pop(lw), vop[e], o[e]);
+          if constexpr (kParts == 3)
+#pragma unroll
+            for (int e = 0; e < NE; ++e) o[e] = M32::mma(pop(ew), vop[e], o[e]);
         }
       };
       {

@@ -61,6 +61,17 @@ constexpr float kMfmaSlack = 8.f;
 // 700, 12 heads: 7.2, 7.1, 7.3, 7.7).
 constexpr int mfma_bufs(int D) { return D == 64 ? 3 : HELM_MFMA_NBUF; }
 
+// 16-bit parts a weight takes into P . V (the vector-ALU kernel multiplied by
+// the fp32 weight).  f16: hi + lo, 22 bits.  bf16: hi + lo are 16 bits and, at
+// the head dims that had the vector-ALU kernel, a third part holds the last
+// eight, so that the fp32 weight enters exactly.  Without it a chunk's outputs
+// were 1.7e-6 off before their rounding, with it 5e-7, as far as fp32 sums in
+// two orders are.  It costs a decode call nothing and a chunk a third more
+// matrix work: D = 256, 512 tokens over 4,700, soft-capped under a window mask,
+// 99 -> 110 us; D = 64, 512 over 16k, 125 -> 146.
+template <typename T>
+constexpr int weight_parts(int D) { return std::is_same<T, bf16_t>::value && D != 128 ? 3 : 2; }
+
 // kFeatMask16: the mask is 16-bit (bf16 / fp16); the decode and 32-row chunk
 // kernels read it at that width (the 16-row chunk kernel at run time)
 enum MfmaFeat { kFeatMask = 1, kFeatCap = 2, kFeatCausal = 4, kFeatMask16 = 8 };
@@ -81,6 +92,14 @@ template <> struct VRow<64> { typedef mf_u32x2 type; };
 template <> struct VRow<128> { typedef mf_u32x4 type; };
 template <> struct VRow<256> { typedef mf_u32x8 type; };
 
+// Low / high 16-bit halves of two words packed into one: (a.lo, b.lo), (a.hi, b.hi).
+__device__ __forceinline__ uint32_t pack_lo(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x05040100u);
+}
+__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);
+}
+
 template <typename T> struct MfmaOps;
 
 template <> struct MfmaOps<bf16_t> {
@@ -94,6 +113,21 @@ template <> struct MfmaOps<bf16_t> {
                                                 uint32_t& lo) {
     hi = pk(w0, w1);
     lo = pk(w0 - __uint_as_float(hi << 16), w1 - __uint_as_float(hi & 0xffff0000u));
+  }
+  // The leading 8 bits of two weights packed into one word; what they leave of
+  // each (exact) stays in w0 and w1.
+  __device__ static __forceinline__ uint32_t lead(float& w0, float& w1) {
+    const uint32_t u0 = __float_as_uint(w0), u1 = __float_as_uint(w1);
+    w0 -= __uint_as_float(u0 & 0xffff0000u);
+    w1 -= __uint_as_float(u1 & 0xffff0000u);
+    return pack_hi(u0, u1);
+  }
+  // Two weights as three such parts: hi + mid + lo is the fp32 weight exactly.
+  __device__ static __forceinline__ void split3(float w0, float w1, uint32_t& hi, uint32_t& mid,
+                                                uint32_t& lo) {
+    hi = lead(w0, w1);
+    mid = lead(w0, w1);
+    lo = pack_hi(__float_as_uint(w0), __float_as_uint(w1));
   }
   __device__ static __forceinline__ uint32_t pk(float a, float b) {
     typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
@@ -207,14 +241,6 @@ __device__ __forceinline__ uint2 ld_tr16(const char* lds_addr) {
   const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
       (__attribute__((address_space(3))) v4i16*)(lds_addr));
   return __builtin_bit_cast(uint2, r);
-}
-
-// Low / high 16-bit halves of two words packed into one: (a.lo, b.lo), (a.hi, b.hi).
-__device__ __forceinline__ uint32_t pack_lo(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_perm(b, a, 0x05040100u);
-}
-__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
 // ---- page records held one per lane ------------------------------------------
@@ -373,9 +399,10 @@ __device__ __forceinline__ void mfma_refresh_max(float bm, float& m, float& lsum
   }
 }
 
-// Weights exp(x - m) of the four tokens into l and, as hi + lo 16-bit parts,
-// P . V into O (V operand v: tokens q4 + 4j at the lane's dims of the row).
-template <class Ops, class V, int NO>
+// Weights exp(x - m) of the four tokens into l and, as PARTS 16-bit parts (2:
+// hi + lo, 3: all 24 bits of a bf16 call's weights), P . V into O (V operand v:
+// tokens q4 + 4j at the lane's dims of the row).
+template <int PARTS, class Ops, class V, int NO>
 __device__ __forceinline__ void mfma_pv(const float (&x)[4], const V (&v)[4], float m,
                                         float& lsum, mf_f32x4 (&o)[NO]) {
   const float base = (m == -INFINITY) ? 0.f : m;
@@ -385,9 +412,14 @@ __device__ __forceinline__ void mfma_pv(const float (&x)[4], const V (&v)[4], fl
     wt[r] = fexp(x[r] - base);
     lsum += wt[r];
   }
-  uint32_t h01, l01, h23, l23;
-  Ops::split2(wt[0], wt[1], h01, l01);
-  Ops::split2(wt[2], wt[3], h23, l23);
+  uint32_t h01, l01, h23, l23, e01 = 0u, e23 = 0u;
+  if constexpr (PARTS == 3) {
+    Ops::split3(wt[0], wt[1], h01, l01, e01);
+    Ops::split3(wt[2], wt[3], h23, l23, e23);
+  } else {
+    Ops::split2(wt[0], wt[1], h01, l01);
+    Ops::split2(wt[2], wt[3], h23, l23);
+  }
   const mf_u32x4 pop = mf_u32x4{h01, h23, l01, l23};
 #pragma unroll
   for (int w = 0; w < NO / 2; ++w) {
@@ -397,11 +429,18 @@ __device__ __forceinline__ void mfma_pv(const float (&x)[4], const V (&v)[4], fl
     const uint32_t b23 = pack_hi(v[2][w], v[3][w]);
     o[2 * w] = Ops::mma(pop, mf_u32x4{a01, a23, a01, a23}, o[2 * w]);
     o[2 * w + 1] = Ops::mma(pop, mf_u32x4{b01, b23, b01, b23}, o[2 * w + 1]);
+    if constexpr (PARTS == 3) {
+      // (the same shape with half of P zero: a 16x16x16 product right after the
+      // 16x16x32 one has read O before its result was there)
+      const mf_u32x4 pex = mf_u32x4{e01, e23, 0u, 0u};
+      o[2 * w] = Ops::mma(pex, mf_u32x4{a01, a23, a01, a23}, o[2 * w]);
+      o[2 * w + 1] = Ops::mma(pex, mf_u32x4{b01, b23, b01, b23}, o[2 * w + 1]);
+    }
   }
 }
 
 // One 16-token block of the recurrence: q . k, logits, max refresh, P . V.
-template <class Ops, bool kMask, bool kCap, bool kCausal, class V, int NK, int NO>
+template <class Ops, int PARTS, bool kMask, bool kCap, bool kCausal, class V, int NK, int NO>
 __device__ __forceinline__ void mfma_block_step(const mf_u32x4 (&k)[NK], const V (&v)[4],
                                                 const float (&mk)[4], int ntok, int tok0,
                                                 const mf_u32x4 (&qop)[NK], float& m, float& lsum,
@@ -411,7 +450,7 @@ __device__ __forceinline__ void mfma_block_step(const mf_u32x4 (&k)[NK], const V
   mfma_logits<kMask, kCap, kCausal>(mfma_qk<Ops>(k, qop), mk, ntok, tok0, scale, cap, inv_cap,
                                     s_vis, q4, x);
   mfma_refresh_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), m, lsum, o, q4);
-  mfma_pv<Ops>(x, v, m, lsum, o);
+  mfma_pv<PARTS, Ops>(x, v, m, lsum, o);
 }
 
 template <class Src> struct LanesOf;
@@ -606,8 +645,8 @@ __device__ __forceinline__ void decode_mfma_body(const AttnParams& p, const Src&
     float mk[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) mk[r] = kMask ? mrow.widen<kMask16>(B.mk[r]) : 0.f;
-    mfma_block_step<Ops, kMask, kCap, kCausal>(B.k, B.v, mk, B.ntok, B.tok0, qop, m, lsum, o,
-                                               scale, cap, inv_cap, s_vis, q4);
+    mfma_block_step<Ops, weight_parts<T>(D), kMask, kCap, kCausal>(
+        B.k, B.v, mk, B.ntok, B.tok0, qop, m, lsum, o, scale, cap, inv_cap, s_vis, q4);
   };
 
   // ---- dynamic block claiming (p.dyn): the waves of every workgroup of the
