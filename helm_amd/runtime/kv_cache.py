@@ -436,6 +436,8 @@ class _AppendQueue:
         n = K.size(2)
         if n == 0:
             return
+        if (V.shape != K.shape or K.size(1) != dst_k.size(1) or K.size(3) != dst_k.size(3)):
+            raise ValueError("tokens must be [1, Hkv, n, D] of the destination's Hkv and D")
         if K.dtype != dst_k.dtype:
             K = K.to(dst_k.dtype)
         if V.dtype != dst_v.dtype:
@@ -747,7 +749,7 @@ class KVCacheManager:
 
     def _queue_contiguous(self, layer_id: int, at: int, K: torch.Tensor, V: torch.Tensor):
         dk, dv = self.cont_K[layer_id], self.cont_V[layer_id]
-        if dk.device.type == "cuda" and K.device.type == "cuda":
+        if dk.device.type == "cuda" and K.device == dk.device and V.device == dk.device:
             self._appends.add(dk, dv, at, K, V)
         else:
             self._appends.flush()
@@ -1266,18 +1268,21 @@ def _decode_mask_args(m: torch.Tensor, device, B: int, Hq: int, t_max: int):
 
 def _decode_operands_plain(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     """True when one native decode call can take the step's query and write its
-    tokens: 16-bit tensors of one dtype on a HIP device, D = 128, one 16-row
+    tokens: 16-bit tensors of one dtype on one HIP device, D = 128, one 16-row
     tile per KV head, dense 16-byte-aligned rows, and no environment switch
-    that asks for another route."""
+    that asks for another route.  (Tokens elsewhere are the general path's,
+    which copies them.)"""
     B, Hq, S, D = q.shape
+    device = q.device
     if (q.dtype not in _KV16 or S != 1 or D != 128 or B > _native.DECODE_MAX_SEQS
-            or not q.is_cuda or k.dtype is not q.dtype or v.dtype is not q.dtype
-            or not q.is_contiguous()):
+            or not q.is_cuda or k.device != device or v.device != device
+            or k.dtype is not q.dtype or v.dtype is not q.dtype or not q.is_contiguous()):
         return False
-    kB, Hkv, kS, _ = k.shape
+    kB, Hkv, kS, kD = k.shape
     ks, vs = k.stride(), v.stride()
     if (Hq > 16 * Hkv                           # more than one 16-row tile per KV head
-            or kB < B or kS != 1 or ks[3] != 1 or vs[3] != 1 or ks[1] != vs[1]
+            or kB < B or kS != 1 or kD != D or v.shape != k.shape
+            or ks[3] != 1 or vs[3] != 1 or ks[1] != vs[1]
             or (ks[1] * 2) % 16
             or (k.data_ptr() | v.data_ptr() | q.data_ptr() | (ks[0] * 2) | (vs[0] * 2)) % 16):
         return False

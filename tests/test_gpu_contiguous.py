@@ -181,3 +181,32 @@ def test_contiguous_step_one_call_equals_two(dtype, Hq, Hkv, D, layout, n, monke
     for b in range(B):
         assert torch.equal(got[0][1 + b][0, :, n], kn[b, :, 0])
         assert torch.equal(got[0][1 + b][1, :, n], vn[b, :, 0])
+
+
+@pytest.mark.parametrize("where", ["both", "k", "v"])
+@pytest.mark.parametrize("contiguous", [True, False])
+def test_tokens_on_the_host_are_copied(where, contiguous):
+    """A decode step whose new tokens live on the CPU: the same result and the
+    same cache contents as with the tokens on the device."""
+    B, Hq, Hkv, D, T, dtype = 2, 32, 8, 128, 70, torch.bfloat16
+    g = torch.Generator().manual_seed(9)
+    q = torch.randn(B, Hq, 1, D, generator=g).to(dtype).to(DEV)
+    k, v, kn, vn = (torch.randn(B, Hkv, n, D, generator=g).to(dtype) for n in (T, T, 1, 1))
+    outs = []
+    for host in (False, True):
+        mgrs = [KVCacheManager(KVAllocator(1, Hkv, D, page_size=16, dtype=dtype),
+                               gpu_high_watermark_bytes=10 ** 12) for _ in range(B)]
+        for b, m in enumerate(mgrs):
+            if contiguous:
+                assert m.build_contiguous(1, Hkv, D, 128, DEV, dtype)
+                m.prefill_contiguous(0, k[b:b + 1].to(DEV), v[b:b + 1].to(DEV))
+            else:
+                m.append_prefill(0, k[b:b + 1].to(DEV), v[b:b + 1].to(DEV))
+        a = kn if host and where in ("both", "k") else kn.to(DEV)
+        c = vn if host and where in ("both", "v") else vn.to(DEV)
+        outs.append(_decode_batched(mgrs, q, a, c, 0, 1 / math.sqrt(D)).cpu())
+        if contiguous:
+            for b, m in enumerate(mgrs):
+                assert torch.equal(m.cont_K[0][0, :, T:T + 1].cpu(), kn[b])
+                assert torch.equal(m.cont_V[0][0, :, T:T + 1].cpu(), vn[b])
+    assert torch.equal(outs[0], outs[1])
