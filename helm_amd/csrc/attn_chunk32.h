@@ -550,7 +550,8 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
             Ops::split3(w0, w1, hw[q], lw[q], ew[q]);
           } else if constexpr (kParts == 2) {
             lsum += w0 + w1;
-            Ops::split2(w0, w1, hw[q], lw[q]);
+            if constexpr (std::is_same<T, f16_t>::value) Ops::split2_mix(w0, w1, hw[q], lw[q]);
+            else Ops::split2(w0, w1, hw[q], lw[q]);
           } else {
             hw[q] = Ops::pk(w0, w1);
             lsum = dot2<T>(hw[q], Ops::ones8()[0], lsum);

@@ -161,15 +161,22 @@ template <> struct MfmaOps<f16_t> {
     typedef float f2 __attribute__((ext_vector_type(2)));
     const h2 h = __builtin_convertvector((f2){w0, w1}, h2);
     hi = __builtin_bit_cast(uint32_t, h);
-    // w - hi, exact: v_fma_mix_f32 reads the f16 half in place (the compiler
-    // would convert each half to fp32 first, one more instruction per weight;
-    // D = 64 chunk of 777 over 2,777, 14 / 2 heads: 30.1 -> 29.2 us)
-    f2 r;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r[0]) : "v"(hi), "v"(w0));
+    const f2 back = __builtin_convertvector(h, f2);
+    lo = pk(w0 - back[0], w1 - back[1]);
+  }
+  // The same with w - hi (exact) by v_fma_mix_f32, which reads the f16 half in
+  // place: one conversion less per weight (D = 64 chunk of 777 over 2,777,
+  // 14 / 2 heads: 30.1 -> 29.2 us).  Not in the decode kernel, where the asm
+  // holds the scheduler back (D = 128, 2,048 tokens: 8.07 us, with it 8.12).
+  __device__ static __forceinline__ void split2_mix(float w0, float w1, uint32_t& hi,
+                                                    uint32_t& lo) {
+    hi = pk(w0, w1);
+    float r0, r1;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hi), "v"(w0));
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-        : "=v"(r[1])
+        : "=v"(r1)
         : "v"(hi), "v"(w1));
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, h2));
+    lo = pk(r0, r1);
   }
 };
 
