@@ -436,8 +436,6 @@ class _AppendQueue:
         n = K.size(2)
         if n == 0:
             return
-        if (V.shape != K.shape or K.size(1) != dst_k.size(1) or K.size(3) != dst_k.size(3)):
-            raise ValueError("tokens must be [1, Hkv, n, D] of the destination's Hkv and D")
         if K.dtype != dst_k.dtype:
             K = K.to(dst_k.dtype)
         if V.dtype != dst_v.dtype:
@@ -749,7 +747,8 @@ class KVCacheManager:
 
     def _queue_contiguous(self, layer_id: int, at: int, K: torch.Tensor, V: torch.Tensor):
         dk, dv = self.cont_K[layer_id], self.cont_V[layer_id]
-        if dk.device.type == "cuda" and K.device == dk.device and V.device == dk.device:
+        dev = dk.device
+        if dk.is_cuda and K.device == dev and V.device == dev:
             self._appends.add(dk, dv, at, K, V)
         else:
             self._appends.flush()
