@@ -116,6 +116,8 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   static_assert(NW == 4 || NW == 8, "waves per workgroup");
   constexpr int SB = kChunkStage;   // 16-token blocks per stage
   constexpr int kParts = chunk32_parts<T>(D);
+  constexpr int kShift = weight_shift<T>(D);
+  constexpr float kSlack = chunk_slack(kShift), kUnit = 1.f / (1 << kShift);
   constexpr bool kAhead = !((FEAT & kFeatMask) && D == 256);
   constexpr int NK = D / 16;        // 16-dim steps of q . k
   constexpr int NE = D / 32;        // 32-dim groups of P . V
@@ -524,9 +526,11 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
         float bm = x[0];
 #pragma unroll
         for (int r = 1; r < 16; ++r) bm = fmaxf(bm, x[r]);
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(bm > m + kMfmaSlack) != 0, 0)) {
-          // refresh the row max (both halves of the row agree)
-          const float mn = fmaxf(m, fmaxf(bm, __shfl_xor(bm, 32, 64)));
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(bm > m + kSlack) != 0, 0)) {
+          // refresh the row max (both halves of the row agree); with scaled
+          // weights to the integer above, so that m - kShift is exact
+          float mn = fmaxf(m, fmaxf(bm, __shfl_xor(bm, 32, 64)));
+          if constexpr (kShift) mn = ceilf(mn);
           const float a = sexp(m - ((mn == -INFINITY) ? 0.f : mn));
           lsum *= a;
           m = mn;
@@ -540,16 +544,17 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
               for (int e = 0; e < NE; ++e) o[e][4 * g + t] *= ar;
             }
         }
-        const float base = (m == -INFINITY) ? 0.f : m;
+        const float base = (m == -INFINITY) ? 0.f : m - kShift;
         uint32_t hw[8], lw[8], ew[8];
+        float ws[8];   // (weights below an ulp of the row's sum add up first)
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
           const float w0 = sexp(x[2 * q] - base), w1 = sexp(x[2 * q + 1] - base);
           if constexpr (kParts == 3) {
-            lsum += w0 + w1;
+            ws[q] = w0 + w1;
             Ops::split3(w0, w1, hw[q], lw[q], ew[q]);
           } else if constexpr (kParts == 2) {
-            lsum += w0 + w1;
+            ws[q] = w0 + w1;
             if constexpr (std::is_same<T, f16_t>::value) Ops::split2_mix(w0, w1, hw[q], lw[q]);
             else Ops::split2(w0, w1, hw[q], lw[q]);
           } else {
@@ -557,6 +562,8 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
             lsum = dot2<T>(hw[q], Ops::ones8()[0], lsum);
           }
         }
+        if constexpr (kParts >= 2)
+          lsum += ((ws[0] + ws[1]) + (ws[2] + ws[3])) + ((ws[4] + ws[5]) + (ws[6] + ws[7]));
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           auto pop = [&](const uint32_t (&w)[8]) {
@@ -615,7 +622,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   }
 
   if (!wave_rows) return;
-  const float lrow = lsum + __shfl_xor(lsum, 32, 64);   // row jr's sum
+  const float lrow = (lsum + __shfl_xor(lsum, 32, 64)) * kUnit;   // row jr's sum
   if (p.direct_out) {
     // the call's only split: normalized rows straight to the output
     // (HELM's final out / max(sum, 1e-12), kv_cache.py:554-555)
@@ -624,7 +631,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const int i = 8 * g + 4 * hh + t;
-        const float inv = 1.f / fmaxf(__shfl(lrow, i, 64), 1e-12f);
+        const float inv = kUnit / fmaxf(__shfl(lrow, i, 64), 1e-12f);
         if (i < nrows)
 #pragma unroll
           for (int e = 0; e < NE; ++e)
@@ -647,7 +654,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
       if (i < nrows) {
         float* dst = &p.ws_o[part_row(i) * D + jr];
 #pragma unroll
-        for (int e = 0; e < NE; ++e) dst[32 * e] = o[e][4 * g + t];
+        for (int e = 0; e < NE; ++e) dst[32 * e] = o[e][4 * g + t] * kUnit;
       }
     }
 }

@@ -72,6 +72,20 @@ constexpr int mfma_bufs(int D) { return D == 64 ? 3 : HELM_MFMA_NBUF; }
 template <typename T>
 constexpr int weight_parts(int D) { return std::is_same<T, bf16_t>::value && D != 128 ? 3 : 2; }
 
+// f16 parts have a floor: what is below 2^-25 is lost.  At head dims 64 and 256
+// (the vector-ALU kernel had no floor) f16 weights are taken times 2^9 and the
+// row's reference max is refreshed once a weight passes 2^6, together below
+// f16's 2^16: the floor lies at 2^-34 of the largest weight, where a million
+// tokens at the floor weigh 2^-14 of the row.  (One key 17 nats above 65,536
+// others, with the floor at 2^-25: the others, 2.7e-3 of the row, counted in its
+// sum and not in its output.)  Chunk of 777 over 2,777, 14 / 2 heads, D = 64:
+// 29.4 us without, 29.3 with; 2^11 and a refresh at 2^4 30.0.
+template <typename T>
+constexpr int weight_shift(int D) { return std::is_same<T, f16_t>::value && D != 128 ? 9 : 0; }
+// the refresh threshold that goes with it, in base-2 units / in natural units
+constexpr float chunk_slack(int shift) { return shift ? 6.f : 8.f; }
+constexpr float decode_slack(int shift) { return shift ? 4.1588831f : kMfmaSlack; }   // 6 ln 2
+
 // kFeatMask16: the mask is 16-bit (bf16 / fp16); the decode and 32-row chunk
 // kernels read it at that width (the 16-row chunk kernel at run time)
 enum MfmaFeat { kFeatMask = 1, kFeatCap = 2, kFeatCausal = 4, kFeatMask16 = 8 };
@@ -385,10 +399,10 @@ __device__ __forceinline__ void mfma_logits(mf_f32x4 sc, const float (&mk)[4], i
 // The lazy online-softmax reference update for a block max bm: when bm
 // exceeds the row max by more than the slack anywhere in the wave, the row
 // max is refreshed and l and the O rows rescaled.
-template <int NO>
+template <int SHIFT, int NO>
 __device__ __forceinline__ void mfma_refresh_max(float bm, float& m, float& lsum,
                                                  mf_f32x4 (&o)[NO], int q4) {
-  if (__builtin_amdgcn_ballot_w64(bm > m + kMfmaSlack)) {
+  if (__builtin_amdgcn_ballot_w64(bm > m + decode_slack(SHIFT))) {
     // refresh the row max (uniform across the row's four lanes)
     float rm = fmaxf(bm, __shfl_xor(bm, 16, 64));
     rm = fmaxf(rm, __shfl_xor(rm, 32, 64));
@@ -409,7 +423,7 @@ __device__ __forceinline__ void mfma_refresh_max(float bm, float& m, float& lsum
 // Weights exp(x - m) of the four tokens into l and, as PARTS 16-bit parts (2:
 // hi + lo, 3: all 24 bits of a bf16 call's weights), P . V into O (V operand v:
 // tokens q4 + 4j at the lane's dims of the row).
-template <int PARTS, class Ops, class V, int NO>
+template <int PARTS, int SHIFT, class Ops, class V, int NO>
 __device__ __forceinline__ void mfma_pv(const float (&x)[4], const V (&v)[4], float m,
                                         float& lsum, mf_f32x4 (&o)[NO]) {
   const float base = (m == -INFINITY) ? 0.f : m;
@@ -417,8 +431,11 @@ __device__ __forceinline__ void mfma_pv(const float (&x)[4], const V (&v)[4], fl
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     wt[r] = fexp(x[r] - base);
-    lsum += wt[r];
+    if constexpr (SHIFT) wt[r] *= static_cast<float>(1 << SHIFT);
+    if constexpr (!(SHIFT || PARTS == 3)) lsum += wt[r];
   }
+  // (the block's sum first: weights below an ulp of the row's sum add up)
+  if constexpr (SHIFT || PARTS == 3) lsum += (wt[0] + wt[1]) + (wt[2] + wt[3]);
   uint32_t h01, l01, h23, l23, e01 = 0u, e23 = 0u;
   if constexpr (PARTS == 3) {
     Ops::split3(wt[0], wt[1], h01, l01, e01);
@@ -447,7 +464,8 @@ __device__ __forceinline__ void mfma_pv(const float (&x)[4], const V (&v)[4], fl
 }
 
 // One 16-token block of the recurrence: q . k, logits, max refresh, P . V.
-template <class Ops, int PARTS, bool kMask, bool kCap, bool kCausal, class V, int NK, int NO>
+template <class Ops, int PARTS, int SHIFT, bool kMask, bool kCap, bool kCausal, class V, int NK,
+          int NO>
 __device__ __forceinline__ void mfma_block_step(const mf_u32x4 (&k)[NK], const V (&v)[4],
                                                 const float (&mk)[4], int ntok, int tok0,
                                                 const mf_u32x4 (&qop)[NK], float& m, float& lsum,
@@ -456,8 +474,8 @@ __device__ __forceinline__ void mfma_block_step(const mf_u32x4 (&k)[NK], const V
   float x[4];
   mfma_logits<kMask, kCap, kCausal>(mfma_qk<Ops>(k, qop), mk, ntok, tok0, scale, cap, inv_cap,
                                     s_vis, q4, x);
-  mfma_refresh_max(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), m, lsum, o, q4);
-  mfma_pv<PARTS, Ops>(x, v, m, lsum, o);
+  mfma_refresh_max<SHIFT>(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), m, lsum, o, q4);
+  mfma_pv<PARTS, SHIFT, Ops>(x, v, m, lsum, o);
 }
 
 template <class Src> struct LanesOf;
@@ -652,7 +670,7 @@ __device__ __forceinline__ void decode_mfma_body(const AttnParams& p, const Src&
     float mk[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) mk[r] = kMask ? mrow.widen<kMask16>(B.mk[r]) : 0.f;
-    mfma_block_step<Ops, weight_parts<T>(D), kMask, kCap, kCausal>(
+    mfma_block_step<Ops, weight_parts<T>(D), weight_shift<T>(D), kMask, kCap, kCausal>(
         B.k, B.v, mk, B.ntok, B.tok0, qop, m, lsum, o, scale, cap, inv_cap, s_vis, q4);
   };
 
@@ -832,6 +850,14 @@ __device__ __forceinline__ void decode_mfma_body(const AttnParams& p, const Src&
   }
 
   // ---- per-wave state to LDS ---------------------------------------------------
+  if constexpr (weight_shift<T>(D) != 0) {   // the weights' scale taken back (exact)
+    constexpr float kUnit = 1.f / (1 << weight_shift<T>(D));
+    lsum *= kUnit;
+#pragma unroll
+    for (int e = 0; e < NO; ++e)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[e][r] *= kUnit;
+  }
   float lrow = lsum + __shfl_xor(lsum, 16, 64);
   lrow += __shfl_xor(lrow, 32, 64);
   if (q4 == 0) {
@@ -1098,7 +1124,7 @@ __global__ __launch_bounds__(256) void chunk_mfma_kernel(AttnParams p, Src src) 
           mfma_logits<kMask, kCap, kCausal>(mfma_qk<Ops>(k, qop), mk, sv_cur.ntok[j],
                                             sv_cur.tok0[j], scale, cap, inv_cap, s_vis, q4, x[h]);
         }
-        mfma_refresh_max(fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
+        mfma_refresh_max<0>(fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
                                fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3]))),
                          m, lsum, o, q4);
         const float base = (m == -INFINITY) ? 0.f : m;

@@ -50,3 +50,42 @@ def test_bf16_weights_keep_all_their_bits(D, S):
     out = perform_streaming_attention(q.to(DEV), _pages(K, V, [3]),
                                       attention_mask=_zero_mask(S, 3))
     assert (out[0].double().cpu() - ref).abs().max().item() <= 8 * 2.0 ** -24
+
+
+def _one_dominant_key(D, S, gap, T, V, pps, monkeypatch):
+    """(f16 attention, the float64 result) of S query rows over T + 1 keys in
+    pages of 64: the first key's logit is `gap`, every other's 0.  V [2, T + 1, D]."""
+    monkeypatch.setenv("HELM_AMD_PPS", str(pps))
+    K = torch.zeros(1, 2, T + 1, D, dtype=torch.float16)
+    K[:, :, 0, 0] = gap
+    q = torch.zeros(1, 4, S, D, dtype=torch.float16)
+    q[..., 0] = math.sqrt(D)
+    sizes = [64] * (T // 64) + [T % 64 + 1]
+    out = perform_streaming_attention(q.to(DEV), _pages(K, V[None], sizes),
+                                      attention_mask=_zero_mask(S, T + 1))[0].double().cpu()
+    w = torch.full((T + 1,), math.exp(-gap), dtype=torch.float64)
+    w[0] = 1
+    ref = (w / w.sum()) @ V.double()                              # [2, D]
+    return out, ref.repeat_interleave(2, 0)[:, None].expand(4, S, D)
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("S,T", [(1, 8000), (40, 65536)])       # decode, chunk: one split
+@pytest.mark.parametrize("gap", [16.5, 17.0, 18.0])
+@pytest.mark.parametrize("values", ["ones", "one_two", "sink_zero", "random"])
+def test_f16_keys_far_below_one_dominant_key(D, S, T, gap, values, monkeypatch):
+    """Many keys that together weigh 1e-4 to 4e-3 of the row, each below 2^-23 of
+    the largest weight (the ones' sum: also below an ulp of the row's).  The output is off by its own rounding (2^-11 relative,
+    half an ulp, and 2^-25 where it is subnormal), the weights' floor (2^-34 each)
+    and 1e-6 of fp32 rounding."""
+    g = torch.Generator().manual_seed(D + S)
+    V = torch.ones(2, T + 1, D, dtype=torch.float16)
+    if values == "one_two":
+        V[:, 1:] = 2
+    elif values == "sink_zero":
+        V[:, 0] = 0
+    elif values == "random":
+        V = torch.randn(2, T + 1, D, generator=g).half()
+    out, ref = _one_dominant_key(D, S, gap, T, V, 128 if S == 1 else 1025, monkeypatch)
+    bound = ref.abs() * 2.0 ** -11 + 2.0 ** -25 + T * 2.0 ** -34 * V.abs().max() + 1e-6 * ref.abs()
+    assert ((out - ref).abs() <= bound).all(), ((out - ref).abs() / bound).max().item()
