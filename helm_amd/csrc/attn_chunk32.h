@@ -622,6 +622,33 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   }
 
   if (!wave_rows) return;
+  if constexpr (D != 128) {
+    if (__builtin_expect(any_nan<NE>(o), 0)) {
+      // everything uniform is read from the kernel arguments again: kept in
+      // scalar registers for this rare path it spilled others in the loop
+      // (D = 256, 512 over 4,700, soft-capped under a window: 105.1 us without the
+      // path, 106.7 with it, 108.0 with the arguments kept)
+      const KernelArgs<Src> ka;
+      const AttnParams& pc = ka.p();
+      const Src& sc = ka.src();
+      const int hkc = blockIdx.y % pc.Hkv;
+      const int lo_c = min(pc.lo, sc.n_pages(blockIdx.z));
+      const int first = lo_c + (int)blockIdx.x * pc.pps;
+      const int last = min(min(pc.hi, sc.n_pages(blockIdx.z)), first + pc.pps);
+      const int row0 = (query_block(pc) * NW + (int)(threadIdx.x >> 6)) * kChunk32Rows;
+      const RowCoord rw = row_coord(row0 + (row0 + jr < pc.G * pc.S ? jr : 0), pc.G);
+      infinite_values<T, Src, FEAT, D>(
+          pc, sc, blockIdx.z, hkc, first, 0, (last - first) * pc.bpp, 1, rw.g, rw.s, m * kLn2, lane,
+          [&](float w, const uint16_t* v) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const float wr = __shfl(w, 8 * (r >> 2) + 4 * hh + (r & 3), 64);
+#pragma unroll
+              for (int e = 0; e < NE; ++e) o[e][r] = with_infinite<T>(o[e][r], wr, v[32 * e + jr]);
+            }
+          });
+    }
+  }
   const float lrow = (lsum + __shfl_xor(lsum, 32, 64)) * kUnit;   // row jr's sum
   if (p.direct_out) {
     // the call's only split: normalized rows straight to the output

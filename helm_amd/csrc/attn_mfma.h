@@ -478,6 +478,107 @@ __device__ __forceinline__ void mfma_block_step(const mf_u32x4 (&k)[NK], const V
   mfma_pv<PARTS, SHIFT, Ops>(x, v, m, lsum, o);
 }
 
+// True where any O of the wave is NaN.
+template <int NO, class O>
+__device__ __forceinline__ bool any_nan(const O (&o)[NO]) {
+  float t = 0.f;
+#pragma unroll
+  for (int e = 0; e < NO; ++e)
+#pragma unroll
+    for (int r = 0; r < (int)(sizeof(O) / 4); ++r) t = fmaf(o[e][r], 0.f, t);
+  return __builtin_amdgcn_ballot_w64(!(t == 0.f)) != 0;
+}
+
+// The arguments of a kernel (AttnParams p, Src src), read again from where the
+// launch put them: a rare path that goes through here keeps none of them in
+// registers beside the loop before it.
+template <class Src>
+struct KernelArgs {
+  const char* base;
+  __device__ __forceinline__ KernelArgs() {
+    auto ka = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));
+    base = (const char*)ka;
+  }
+  __device__ __forceinline__ const AttnParams& p() const {
+    return *reinterpret_cast<const AttnParams*>(base);
+  }
+  __device__ __forceinline__ const Src& src() const {
+    constexpr size_t at = (sizeof(AttnParams) + alignof(Src) - 1) / alignof(Src) * alignof(Src);
+    return *reinterpret_cast<const Src*>(base + at);
+  }
+};
+
+// Infinite values.  A weight times an infinite value is infinite, but the sum
+// of its 16-bit parts' products is NaN where a part is zero or of the other
+// sign (1.0 has hi = 1, lo = 0).  At the head dims that had the vector-ALU kernel
+// a wave whose O holds a NaN at the end of its walk comes here, a rare path
+// kept short and out of the loop (a second walk with parts above zero instead
+// slowed the chunks by 2 to 7% and the soft-capped decode by 8%): it looks
+// through V of the wave's blocks (blk, blk + step, ...) again and, per token
+// with an infinity or NaN, takes the weight of each row in fp32, from the same
+// logit and the row's final max m (natural units, row (g, s) in this lane), and
+// hands it with the token's V row to add, which corrects O with the fp32 product.
+template <typename T, class Src, int FEAT, int D, class Add>
+__device__ __forceinline__ void infinite_values(const AttnParams& p, const Src& src, int b, int hk,
+                                                int pg0, int blk, int nblk, int step, int g, int s,
+                                                float m, int lane, Add&& add) {
+  constexpr int kRow = 2 * D;
+  constexpr uint32_t kExp = std::is_same<T, bf16_t>::value ? 0x7f80u : 0x7c00u;
+  const int h = hk * p.G + g;
+  const char* qp = reinterpret_cast<const char*>(p.q) + ((int64_t)(b * p.Hq + h) * p.S + s) * kRow;
+  const float base = (m == -INFINITY) ? 0.f : m;
+#pragma unroll 1
+  for (; blk < nblk; blk += step) {
+    const int pi = blk / p.bpp;
+    const int tok_in = (blk - pi * p.bpp) * kBlockTok;
+    const PageView pv = src.page(b, pg0 + pi, hk);
+    const int ntok = sclamp(pv.used - tok_in, 0, kBlockTok);
+    const char* vb = pv.v + tok_in * kRow;
+    const auto rv = make_rsrc(vb, ntok * kRow);
+    bool bad = false;
+#pragma unroll
+    for (int c = 0; c < kBlockTok * kRow / 1024; ++c) {
+      const mf_u32x4 v = buf_load16_nt(rv, 1024 * c + 16 * lane);   // (zero past the tokens)
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+        bad = bad || (v[w] & kExp) == kExp || ((v[w] >> 16) & kExp) == kExp;
+    }
+    if (!__builtin_amdgcn_ballot_w64(bad)) continue;
+#pragma unroll 1
+    for (int t = 0; t < ntok; ++t) {
+      const char* kp = pv.k + (tok_in + t) * kRow;
+      float x = 0.f;
+#pragma unroll 1
+      for (int i = 0; i < kRow; i += 4)
+        x = dot2<T>(*reinterpret_cast<const uint32_t*>(qp + i),
+                    *reinterpret_cast<const uint32_t*>(kp + i), x);
+      x *= p.scale;
+      // (tanh to 1e-6: only whether the weight is zero matters)
+      if constexpr ((FEAT & kFeatCap) != 0)
+        x = (1.f - 2.f / (fexp(2.f * x / p.softcap) + 1.f)) * p.softcap;
+      const int tok = pv.tok_off + tok_in + t;
+      if constexpr ((FEAT & kFeatMask) != 0) x += mask_row(p, b, h, s)[tok];
+      if constexpr ((FEAT & kFeatCausal) != 0)
+        if (tok > s + p.causal - 1) x = -INFINITY;
+      add(fexp(x - base), reinterpret_cast<const uint16_t*>(vb + t * kRow));
+    }
+  }
+}
+
+// O with the product of weight w and value bits v: left alone where it or v is
+// finite; the NaN of the parts' products (any but `done`) gives way to w v.
+template <typename T>
+__device__ __forceinline__ float with_infinite(float o, float w, uint16_t v) {
+  constexpr uint32_t kDone = 0x7fc0dead;   // a NaN that stays
+  Raw<2> raw;
+  raw.w[0] = v;
+  const float term = w * elem_f32<T>(raw, 0);
+  if (fabsf(o) < INFINITY || fabsf(elem_f32<T>(raw, 0)) < INFINITY) return o;
+  const float sum = (o != o && __float_as_uint(o) != kDone) ? term : o + term;
+  return sum != sum ? __uint_as_float(kDone) : sum;
+}
+
 template <class Src> struct LanesOf;
 template <> struct LanesOf<PoolSrc> { using type = PoolLanes; };
 template <> struct LanesOf<DescSrc> { using type = DescLanes; };
@@ -846,6 +947,21 @@ __device__ __forceinline__ void decode_mfma_body(const AttnParams& p, const Src&
       if (k + u >= nmine) break;
       load_block(wave + (k + u + NB - 1) * NW, buf[(u + NB - 1) % NB]);
       compute_block(buf[u]);
+    }
+    if constexpr (D != 128) {
+      if (__builtin_expect(any_nan<NO>(o), 0))
+        infinite_values<T, Src, FEAT, D>(
+            p, src, b, hk, pg0, wave, nblk, NW, g_row, s_row, m, lane,
+            [&](float w, const uint16_t* v) {
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const float wr = __shfl(w, 4 * q4 + r, 64);
+#pragma unroll
+                for (int e = 0; e < NO; ++e)
+                  o[e][r] = with_infinite<T>(
+                      o[e][r], wr, v[(D == 64 ? 4 : 8) * n + (e >> 3) * 128 + (e & 7)]);
+              }
+            });
     }
   }
 

@@ -6,9 +6,11 @@ import pytest
 import torch
 
 from helm_amd.runtime.kv_cache import KVPage, perform_streaming_attention
+from oracle import attention as A
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda:0")
+TOL = {torch.float16: 2e-3, torch.bfloat16: 1e-2}
 
 
 def _pages(K, V, sizes):
@@ -89,3 +91,29 @@ def test_f16_keys_far_below_one_dominant_key(D, S, T, gap, values, monkeypatch):
     out, ref = _one_dominant_key(D, S, gap, T, V, 128 if S == 1 else 1025, monkeypatch)
     bound = ref.abs() * 2.0 ** -11 + 2.0 ** -25 + T * 2.0 ** -34 * V.abs().max() + 1e-6 * ref.abs()
     assert ((out - ref).abs() <= bound).all(), ((out - ref).abs() / bound).max().item()
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S,sizes", [(1, [16, 16, 7]), (1, [64] * 40), (40, [16, 16, 7]),
+                                     (40, [64] * 40), (150, [48] * 30 + [9])])
+def test_infinite_values(D, dtype, S, sizes):
+    """Infinities in V come out as the fp32 weights give them: +inf, -inf, NaN
+    where both signs meet, also under a weight of e^-40; the other columns keep
+    their values (tolerance: the output's rounding, as without infinities)."""
+    T = sum(sizes)
+    g = torch.Generator().manual_seed(D + S + T)
+    K, V = (torch.randn(1, 2, T, D, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(1, 6, S, D, generator=g).to(dtype)
+    q[..., 0] = 4
+    K[:, :, 13] = 0
+    K[:, :, 13, 0] = -10 * math.sqrt(D)
+    V[:, :, 5, 0] = V[:, :, 9, 2] = V[:, :, 13, 3] = math.inf
+    V[:, :, 7, 1] = V[:, :, 11, 2] = -math.inf
+    out = perform_streaming_attention(q.to(DEV), _pages(K, V, sizes),
+                                      attention_mask=_zero_mask(S, T))[0].double().cpu()
+    assert (out[..., 0] == math.inf).all() and (out[..., 1] == -math.inf).all()
+    assert out[..., 2].isnan().all() and (out[..., 3] == math.inf).all()
+    V[..., :4] = 0
+    ref = A.attention_fp64_batched(q[0], K[0], V[0])
+    assert (out[..., 4:] - ref[..., 4:]).abs().max().item() <= TOL[dtype]
