@@ -501,12 +501,21 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
           for (int r = 0; r < 16; ++r) x[r] = sc[r] * scale2;
         }
         // finfo.min masks stay finite, as in natural units (a row masked
-        // everywhere gets equal weights, as HELM's loop gives it)
-        if constexpr (kMask)
+        // everywhere gets equal weights, as HELM's loop gives it).  At
+        // D = 64 and 256 (as the vector-ALU kernel): NaN stays, and -inf hides a key, also
+        // where it leaves a row with none; a key masked to -1e30 or below takes
+        // its mask as its logit, as the skipped steps have it: lowered by
+        // 1e30 (log2(e) - 1), so that the masks' order holds across -1e30.
+        if constexpr (kMask && D == 128) {
+          if (add_mask)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) x[r] = fmaxf(fmaf(mk[r], kLog2E, x[r]), -__FLT_MAX__);
+        } else if constexpr (kMask) {
           if (add_mask)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-              x[r] = fmaxf(fmaf(mk[r], kLog2E, x[r]), -__FLT_MAX__);
+              x[r] = mk[r] <= -1e30f ? mk[r] - 0.442695e30f : fmaf(mk[r], kLog2E, x[r]);
+        }
         // the per-token limits, only where a step reaches them (uniform tests):
         // the causal limit when a block's last token is past the wave's first
         // query position, the valid-token limit when a block is partial

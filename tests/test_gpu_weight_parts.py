@@ -117,3 +117,88 @@ def test_infinite_values(D, dtype, S, sizes):
     V[..., :4] = 0
     ref = A.attention_fp64_batched(q[0], K[0], V[0])
     assert (out[..., 4:] - ref[..., 4:]).abs().max().item() <= TOL[dtype]
+
+
+def _chunk(D, dtype, T, S, seed):
+    g = torch.Generator().manual_seed(seed)
+    K, V = (torch.randn(1, 2, T, D, generator=g).to(dtype) for _ in range(2))
+    return (1.5 * torch.randn(1, 4, S, D, generator=g)).to(dtype), K, V
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S", [1, 40])
+@pytest.mark.parametrize("mdtype", ["own", "f32"])
+@pytest.mark.parametrize("cap", [None, 50.0])
+def test_rows_masked_everywhere(D, dtype, S, mdtype, cap):
+    """Rows with no visible key: -inf masks leave a row without keys, zeros (a
+    chunk at D = 128 bounds its logits: the mean of V); finfo.min masks weigh
+    every key alike; -inf beside finfo.min hides."""
+    T = 200
+    q, K, V = _chunk(D, dtype, T, S, D + S)
+    mt = dtype if mdtype == "own" else torch.float32
+    low = torch.finfo(mt).min
+    mask = torch.zeros(1, 4, S, T, dtype=mt)
+    mask[:, 0] = -math.inf
+    mask[:, 1] = low
+    mask[:, 2] = low
+    mask[:, 2, :, ::2] = -math.inf
+    mask[:, 3, :, :T // 2] = -math.inf
+    out = perform_streaming_attention(q.to(DEV), _pages(K, V, [64, 64, 64, 8]), softcap=cap,
+                                      attention_mask=mask.to(DEV))[0].double().cpu()
+    mean = V[0].double().mean(1)
+    keeps = D == 128 and S > 1
+    assert (out[0] - (mean[0] if keeps else 0)).abs().max().item() <= (TOL[dtype] if keeps else 0)
+    exact = A.attention_fp64_batched(q[0], K[0], V[0], mask=mask[0].float(), softcap=cap)
+    # (an f16 finfo.min is no bound: the scores still count)
+    if mt == torch.float16:
+        assert (out[1] - exact[1]).abs().max().item() <= TOL[dtype]
+    else:
+        assert (out[1] - mean[0]).abs().max().item() <= TOL[dtype]
+        want = mean[1] if keeps else V[0, 1, 1::2].double().mean(0)
+        assert (out[2] - want).abs().max().item() <= TOL[dtype]
+    assert (out[3] - exact[3]).abs().max().item() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cap", [None, 50.0])
+@pytest.mark.parametrize("other", [0.0, -1.0])
+def test_nan_keys_under_a_mask_do_not_depend_on_neighbours(D, dtype, cap, other):
+    """A chunk with a NaN key whose mask is zero, its neighbours' masks zero or
+    not: at D = 64 and 256 every row is NaN; at D = 128 the key is left out.  A
+    NaN key under finfo.min is left out at every head dim, also in a step with
+    visible keys."""
+    T, S = 200, 40
+    q, K, V = _chunk(D, dtype, T, S, D + 1)
+    mask = torch.zeros(1, 1, S, T)
+    mask[..., 40:60] = other
+    hidden = mask.clone()
+    hidden[..., 50] = torch.finfo(torch.float32).min
+    ref = A.attention_fp64_batched(q[0], K[0], V[0], mask=hidden[0], softcap=cap)
+    K[:, :, 50] = math.nan
+    mask[..., 50] = 0
+    for m, left_out in ((hidden, True), (mask, D == 128)):
+        out = perform_streaming_attention(q.to(DEV), _pages(K, V, [64, 64, 64, 8]), softcap=cap,
+                                          attention_mask=m.to(DEV))[0].double().cpu()
+        if left_out:
+            assert (out - ref).abs().max().item() <= TOL[dtype]
+        else:
+            assert out.isnan().all()
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("other", [0.0, -1.0])
+def test_infinite_logits_under_a_mask_do_not_depend_on_neighbours(D, other):
+    """Every logit -inf, the masks zero or not: a chunk's rows are zeros at D = 64
+    and 256 and the mean of V at D = 128, where masked logits are bounded."""
+    T, S = 200, 40
+    q, K, V = _chunk(D, torch.bfloat16, T, S, D + 2)
+    q[..., 0] = 1
+    K[..., 0] = -math.inf
+    mask = torch.zeros(1, 1, S, T)
+    mask[..., 20:180] = other
+    out = perform_streaming_attention(q.to(DEV), _pages(K, V, [64, 64, 64, 8]),
+                                      attention_mask=mask.to(DEV))[0].double().cpu()
+    want = V[0].double().mean(1).repeat_interleave(2, 0)[:, None] * (D == 128)
+    assert (out - want).abs().max().item() <= (TOL[torch.bfloat16] if D == 128 else 0)
