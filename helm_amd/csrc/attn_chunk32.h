@@ -501,12 +501,17 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
           for (int r = 0; r < 16; ++r) x[r] = sc[r] * scale2;
         }
         // finfo.min masks stay finite, as in natural units (a row masked
-        // everywhere gets equal weights, as HELM's loop gives it).  At
-        // D = 64 and 256 (as the vector-ALU kernel): NaN stays, and -inf hides a key, also
+        // everywhere gets equal weights, as HELM's loop gives it).  A zero mask
+        // and an added one follow one rule, so that a key's NaN or -inf logit does
+        // not depend on its neighbours' masks.  D = 128 (kBound): every masked
+        // logit is at least -FLT_MAX, NaN and -inf among them (with a zero mask
+        // bounded where the step's maximum asks for it).
+        // Else (as the vector-ALU kernel): NaN stays, and -inf hides a key, also
         // where it leaves a row with none; a key masked to -1e30 or below takes
         // its mask as its logit, as the skipped steps have it: lowered by
         // 1e30 (log2(e) - 1), so that the masks' order holds across -1e30.
-        if constexpr (kMask && D == 128) {
+        constexpr bool kBound = kMask && D == 128;
+        if constexpr (kBound) {
           if (add_mask)
 #pragma unroll
             for (int r = 0; r < 16; ++r) x[r] = fmaxf(fmaf(mk[r], kLog2E, x[r]), -__FLT_MAX__);
@@ -515,6 +520,16 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
 #pragma unroll
             for (int r = 0; r < 16; ++r)
               x[r] = mk[r] <= -1e30f ? mk[r] - 0.442695e30f : fmaf(mk[r], kLog2E, x[r]);
+        }
+        if constexpr (kBound) {
+          float top = x[0];   // (NaN passes through)
+#pragma unroll
+          for (int r = 1; r < 16; ++r) top = __builtin_elementwise_maximum(top, x[r]);
+          // (a token hidden below may stand above the visible ones here)
+          const bool limits = (((bits[K].part | bits[K].limit) >> bp) & 3) != 0;
+          if (__builtin_expect(limits || __builtin_amdgcn_ballot_w64(!(top > -INFINITY)) != 0, 0))
+#pragma unroll
+            for (int r = 0; r < 16; ++r) x[r] = fmaxf(x[r], -__FLT_MAX__);
         }
         // the per-token limits, only where a step reaches them (uniform tests):
         // the causal limit when a block's last token is past the wave's first

@@ -160,7 +160,7 @@ def test_rows_masked_everywhere(D, dtype, S, mdtype, cap):
     assert (out[3] - exact[3]).abs().max().item() <= TOL[dtype]
 
 
-@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("cap", [None, 50.0])
 @pytest.mark.parametrize("other", [0.0, -1.0])
@@ -187,7 +187,7 @@ def test_nan_keys_under_a_mask_do_not_depend_on_neighbours(D, dtype, cap, other)
             assert out.isnan().all()
 
 
-@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("other", [0.0, -1.0])
 def test_infinite_logits_under_a_mask_do_not_depend_on_neighbours(D, other):
     """Every logit -inf, the masks zero or not: a chunk's rows are zeros at D = 64
