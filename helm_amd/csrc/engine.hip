@@ -210,6 +210,7 @@ void settle_fused(Plan& pl, int B, int Hkv) {
       pl.row_waves)
     pl.fused = 0;
   pl.direct = (pl.row_waves && pl.max_splits == 1) ? 1 : 0;
+  if (pl.direct) pl.ml_bytes = pl.o_bytes = 0;   // the kernel writes no partials
 }
 
 // Rows, tiles and the split limits of a kernel choice.
