@@ -306,24 +306,31 @@ int balanced_pps(double pages, double units, int target, int lo_pps, int max_pps
 // 1.6 / 1.0; D = 256 3.3.  A split length from the number of workgroups alone gave
 // 480-workgroup prompts a second split of a few pages and its partials (f16
 // 40 heads, 1,500 tokens: 97 us, one split 47; bf16 8 heads, 4,000 tokens: 85,
-// now 71).
+// now 71).  The merge walks a row's splits, 0.04 us each.  Few KV heads over a long
+// context fill the chip by splits alone (131,072 tokens: 16 / 2 heads, D = 128, 32
+// rows, 64 splits 46.2 us, 128 29.8, 256 31.6; 14 / 2 heads, D = 64, 21 rows, 64
+// splits 45.9, 128 27.3, 256 20.9, 512 25.2): the count is bounded by the shortest
+// split and the kernel's limit only.
 int chunk_pps(const Plan& pl, int D, double units, double rows, double pages, double walk) {
   const double alone = D == 256 ? 3.3 : D == 64 ? 1.6 : pl.nw == 8 ? 2.3 : 2.0;
   const double full = D == 256 ? 3.3 : D == 64 ? 1.0 : pl.nw == 8 ? 2.3 : 1.6;
-  constexpr double kMergeUs = 6.0, kPartialBytesPerUs = 5e6;
+  constexpr double kMergeUs = 6.0, kMergeSplitUs = 0.04, kPartialBytesPerUs = 5e6;
   const double P = std::max(1.0, pages);
   const double cus = device_cus();
   int best_pps = (int)std::ceil(P);
   double best = -1.0;
-  for (int s = 1; s <= 64; ++s) {
+  // (past 64 splits in steps of a 32nd: neighbours differ by less than the estimate)
+  for (int s = 1; s <= max_splits_of(pl); s += std::max(1, s / 32 - 1)) {
     const int pps = (int)std::ceil(P / s);
     // (the workspace query counts on no automatic split being shorter)
     if (s > 1 && pps < min_pps(pl.bpp, kWaves)) break;
     const double n = std::ceil(P / pps);
     const double stages = pps * (double)pl.bpp / kChunkStage;
     const double share = walk > 0.75 ? std::ceil(units * n / cus) : units * n * walk / cus;
-    double us = std::max(stages * alone, share * stages * full);
-    if (n > 1) us += kMergeUs + n * rows * D * 8.0 / kPartialBytesPerUs;
+    const double merge =
+        n > 1 ? kMergeUs + n * (kMergeSplitUs + rows * D * 8.0 / kPartialBytesPerUs) : 0.0;
+    if (best >= 0.0 && merge >= best) break;   // (it only grows)
+    const double us = std::max(stages * alone, share * stages * full) + merge;
     if (best < 0.0 || us < best) {
       best = us;
       best_pps = pps;

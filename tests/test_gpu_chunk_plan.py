@@ -57,3 +57,14 @@ def test_one_split_needs_no_room_for_partials(D, Hq, Hkv, S, T):
     _check(keep, case, 0, T, D, Hkv)
     with pytest.raises(ValueError, match="workspace"):
         _run(args, need - 256)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv,S,least", [(128, 16, 2, 4, 100), (64, 14, 2, 3, 200)])
+def test_few_heads_over_a_long_context_fill_the_chip(D, Hq, Hkv, S, least):
+    """Two KV heads over 131,072 tokens: enough splits for every CU (64 leave
+    half of them or more idle)."""
+    T = 131072
+    args, keep, case = _chunk(D, Hq, Hkv, S, T, seed=D)
+    ws = _run(args, args[-2])
+    assert least <= ws[TICKETS:].view(torch.int32)[0].item() <= 512
+    _check(keep, case, 0, T, D, Hkv)
