@@ -310,31 +310,38 @@ int balanced_pps(double pages, double units, int target, int lo_pps, int max_pps
 // context fill the chip by splits alone (131,072 tokens: 16 / 2 heads, D = 128, 32
 // rows, 64 splits 46.2 us, 128 29.8, 256 31.6; 14 / 2 heads, D = 64, 21 rows, 64
 // splits 45.9, 128 27.3, 256 20.9, 512 25.2): the count is bounded by the shortest
-// split and the kernel's limit only.
-int chunk_pps(const Plan& pl, int D, double units, double rows, double pages, double walk) {
+// split and the kernel's limit only.  pages / max_pages: the mean of the B
+// sequences and what bounds the longest (a split is as long as the longest's
+// needs; the share and the partials are the mean's).
+int chunk_pps(const Plan& pl, int D, int B, double units, double rows, double pages,
+              int max_pages, double walk) {
   const double alone = D == 256 ? 3.3 : D == 64 ? 1.6 : pl.nw == 8 ? 2.3 : 2.0;
   const double full = D == 256 ? 3.3 : D == 64 ? 1.0 : pl.nw == 8 ? 2.3 : 1.6;
   constexpr double kMergeUs = 6.0, kMergeSplitUs = 0.04, kPartialBytesPerUs = 5e6;
-  const double P = std::max(1.0, pages);
+  const double P = std::max(1.0, pages), Pmax = std::max(P, std::min((double)max_pages, P * B));
   const double cus = device_cus();
-  int best_pps = (int)std::ceil(P);
+  const int least = min_pps(pl.bpp, kWaves);
+  int best_pps = (int)std::ceil(Pmax);
   double best = -1.0;
   // (past 64 splits in steps of a 32nd: neighbours differ by less than the estimate)
   for (int s = 1; s <= max_splits_of(pl); s += std::max(1, s / 32 - 1)) {
-    const int pps = (int)std::ceil(P / s);
     // (the workspace query counts on no automatic split being shorter)
-    if (s > 1 && pps < min_pps(pl.bpp, kWaves)) break;
-    const double n = std::ceil(P / pps);
-    const double stages = pps * (double)pl.bpp / kChunkStage;
+    const int pps = std::max((int)std::ceil(Pmax / s), least);
+    // the splits of the mean sequence and of the longest, and their lengths
+    const double n = std::ceil(P / pps), n_max = std::ceil(Pmax / pps);
+    const double stage = (double)pl.bpp / kChunkStage;
+    const double stages = pps * stage, mean_stages = std::min((double)pps, P) * stage;
     const double share = walk > 0.75 ? std::ceil(units * n / cus) : units * n * walk / cus;
     const double merge =
-        n > 1 ? kMergeUs + n * (kMergeSplitUs + rows * D * 8.0 / kPartialBytesPerUs) : 0.0;
+        n_max > 1 ? kMergeUs + n_max * kMergeSplitUs + n * rows * D * 8.0 / kPartialBytesPerUs : 0.0;
     if (best >= 0.0 && merge >= best) break;   // (it only grows)
-    const double us = std::max(stages * alone, share * stages * full) + merge;
+    const double us =
+        std::max(std::min(stages, Pmax * stage) * alone, share * mean_stages * full) + merge;
     if (best < 0.0 || us < best) {
       best = us;
       best_pps = pps;
     }
+    if (pps == least) break;
   }
   return best_pps;
 }
@@ -379,7 +386,8 @@ int make_plan(Plan& pl, int kv_dtype, int q_dtype, int B, int Hq, int Hkv,
   if (pps <= 0 && pl.row_waves == 2 && env_int("HELM_AMD_WG_PER_CU", 0) <= 0) {
     const double tokens = std::max(1.0, avg_pages * max_tok_per_page);
     const double walk = causal ? std::min(1.0, (causal + 0.5 * q_len) / tokens) : 1.0;
-    pps = chunk_pps(pl, D, (double)B * Hkv * pl.qblocks(), (double)B * Hq * q_len, avg_pages, walk);
+    pps = chunk_pps(pl, D, B, (double)B * Hkv * pl.qblocks(), (double)B * Hq * q_len, avg_pages,
+                    max_pages, walk);
   }
   if (pps <= 0) {
     const double units = (double)B * Hkv * pl.qblocks();

@@ -68,3 +68,35 @@ def test_few_heads_over_a_long_context_fill_the_chip(D, Hq, Hkv, S, least):
     ws = _run(args, args[-2])
     assert least <= ws[TICKETS:].view(torch.int32)[0].item() <= 512
     _check(keep, case, 0, T, D, Hkv)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("hint", [True, False])
+def test_ragged_chunks_take_no_split_below_the_shortest(D, hint):
+    """One sequence of 64 pages among 64 of one page, with and without the total
+    page count: splits of at least eight 16-token pages, as the workspace query
+    counts on, and the call fits what it asks for."""
+    lens = [1024] + [16] * 63
+    args, keep, case = _chunk(D, 4, 2, 17, 1024, seed=D, lens=lens,
+                              total_pages=127 if hint else 0)
+    tiles = 2 * 3
+    ws = _run(args, args[-2])
+    counts = ws[TICKETS:].view(torch.int32)[:64 * tiles].view(64, tiles).cpu()
+    assert (counts[0] <= 8).all() and (counts[1:] == 1).all()
+    for b in (0, 1, 63):
+        _check(keep, case, b, lens[b], D, 2)
+
+
+def test_split_length_follows_the_sequence_not_the_table():
+    """One sequence of 100 pages in a table of 4,096 columns, its page count
+    given: the split count of the same call with a table of 100."""
+    counts = []
+    for width in (100, 4096):
+        args, keep, case = _chunk(128, 32, 8, 64, 1600, seed=3, total_pages=100)
+        table = torch.zeros(1, width, dtype=torch.int32, device=DEV)
+        table[:, :100] = case["table"]
+        args[6], args[7], args[15] = table.data_ptr(), width, width
+        ws = _run(args, _native.load().helm_query_workspace_bytes(1, 32, 8, 64, 128, width, 16, 0))
+        counts.append(ws[TICKETS:].view(torch.int32)[0].item())
+        _check(keep, case, 0, 1600, 128, 8)
+    assert counts[0] == counts[1]
