@@ -1,11 +1,15 @@
-"""The matrix-core kernels at head dims 64 and 256 against the float64 oracle.
+"""The matrix-core kernels at head dims 64 and 256 (chunk edges also at 128)
+against the float64 oracle.
 
 The sizes sit at the edges of the kernels' tiles: one row, 16-row decode tiles
 (full, remainder), 32-row chunk waves and 128-row workgroups, 16-token blocks,
 four-block stages, 64-page record windows; one or several splits and both
 merges.  Tolerances: the output's own rounding (half an ulp of the largest
-element, |out| < 4: 2^-9 relative in bf16, 2^-12 in f16) and the weights' hi +
-lo split (2^-16 of sum |w v|, below it): 1e-2 (bf16) and 2e-3 (f16) absolute.
+element, |out| < 4: 2^-9 relative in bf16, 2^-12 in f16): 7.8e-3 and 1e-3
+absolute, with room for the weights' parts (all 24 bits in bf16, 2^-22 and an
+absolute 2^-34 of the largest weight in f16, far below it) and at D = 128 for
+a chunk's weights rounded once (as much again times the spread of V over its
+mean, small against the output's): 1e-2 (bf16) and 2e-3 (f16).
 """
 import math
 
@@ -50,7 +54,7 @@ def _mask(kind, S, T, dtype):
     return m[None, None]
 
 
-@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("Hq,Hkv,S,sizes", [
     (4, 4, 1, [1]),                      # one row, one token
@@ -60,6 +64,8 @@ def _mask(kind, S, T, dtype):
     (4, 2, 17, [16, 16, 11]),            # 34 chunk rows: a full wave and two rows
     (14, 2, 19, [64, 64, 64, 30]),       # 133 rows: a workgroup and five rows
     (4, 1, 150, [16] * 68 + [7]),        # several workgroups, past one record window
+    (4, 2, 40, [48] * 30 + [7]),         # 48-token pages: windows of 64 blocks start mid-page
+    (8, 2, 200, [48] * 30 + [35]),       # the same, several workgroups and a ragged tail
 ])
 @pytest.mark.parametrize("kind,cap", [("none", None), ("causal", None), ("window", None),
                                       ("window", 5.0),      # logits near the cap: tanhf
@@ -83,7 +89,13 @@ def test_streaming_matches_fp64(D, dtype, Hq, Hkv, S, sizes, kind, cap):
             torch.arange(T)[None, :] > torch.arange(S)[:, None], -math.inf)
     ref = A.attention_fp64_batched(q[0], K[0], V[0], softcap=cap,
                                    mask=None if ref_m is None else ref_m[0])
-    err = (out[0].double().cpu() - ref).abs().max().item()
+    diff = (out[0].double().cpu() - ref).abs()
+    if kind == "first_row_masked" and dtype == torch.float16:
+        # f16's finfo.min is -65504: the row's logits, -94,504 in base 2, have an
+        # fp32 ulp of 2^-7, so each weight is off by up to 2^-8 ln 2
+        assert diff[:, 0].max().item() <= TOL[dtype] + 2.0 ** -8 * math.log(2) * V.abs().max().item()
+        diff = diff[:, 1:] if S > 1 else diff * 0
+    err = diff.max().item()
     assert err <= TOL[dtype], err
 
 
