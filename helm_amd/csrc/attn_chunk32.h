@@ -13,7 +13,7 @@
 //
 // Lane l = 32 hh + j (j = l % 32):
 //   q . k   S^T = K Q^T: A = K (row m = token tau(m), dims 16i + 8hh .. + 7),
-//           B = Q^T (column j = query row j), eight MFMAs over the 128 dims.
+//           B = Q^T (column j = query row j), one MFMA per 16 dims.
 //           The result gives lane l, for its query row j, register
 //           r = 4g + t <-> output row m = 8g + 4hh + t, and with
 //           tau(8g + 4h + t) = 16 (g >> 1) + 8h + 4 (g & 1) + t register r holds
@@ -118,6 +118,9 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   constexpr int kParts = chunk32_parts<T>(D);
   constexpr int kShift = weight_shift<T>(D);
   constexpr float kSlack = chunk_slack(kShift), kUnit = 1.f / (1 << kShift);
+  // a window's page records are read one window ahead, except with a mask at
+  // D = 256, whose masks, O and query operand leave no registers for them: there
+  // they are read when the window is entered, once in 64 blocks
   constexpr bool kAhead = !((FEAT & kFeatMask) && D == 256);
   constexpr int NK = D / 16;        // 16-dim steps of q . k
   constexpr int NE = D / 32;        // 32-dim groups of P . V
@@ -255,8 +258,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   // workgroup.  A stage then takes its four blocks' bits and one address by
   // v_readlane, where walking pages and sub-blocks in scalar code took ~120
   // scalar instructions per stage of every wave's serial path (bf16 512 tokens
-  // over 32k: 296 -> 271; D = 64, 512 over 16k: 144 -> 128 us).  The next
-  // window's records are read one window ahead.
+  // over 32k: 296 -> 271; D = 64, 512 over 16k: 144 -> 128 us).
   struct Window {
     uint32_t klo, khi, vlo, vhi;
     int nt, t0;
@@ -379,8 +381,8 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
   // masks; D = 128 soft-capped), at the stage's start before the next stage's
   // K / V: a load after those would have to wait for them too.  Element loads of every step, converted and added
   // even where zero, had bound the masked chunk (bf16 512 over 8,192 tokens under
-  // a 4,096-token window, 32 / 8 heads: 187 us, now 108; D = 256, 512 over 4,700,
-  // soft-capped: 203, now 99).
+  // a 4,096-token window, 32 / 8 heads: 187 us, now 109; D = 256, 512 over 4,700,
+  // soft-capped: 203, now 108).
   typedef typename std::conditional<kMask16, mf_u32x4, mf_u32x8>::type MaskWords;
   constexpr bool kMaskAhead = kMask16 && !(kCap && D == 128);
   MaskWords mkw[kMaskAhead ? 2 : 1][SB];
@@ -471,7 +473,7 @@ __device__ __forceinline__ void chunk32_mfma_body(const AttnParams& p, const Src
 #pragma unroll
         for (int r = 0; r < 16; ++r) sc[r] = 0.f;
         // every K operand read issued before the first MFMA (one LDS wait,
-        // then the eight MFMAs back to back), registers allowing: with a mask
+        // then the MFMAs back to back), registers allowing: with a mask
         // operand its prefetched values take them, and the compiler's order
         // stays
         mf_u32x4 ka[NK];
@@ -719,8 +721,8 @@ __global__ __launch_bounds__(NW * 64, 2) void chunk32_mfma_kernel(AttnParams p, 
 // 32 x 256 query operand take 192 registers before any score: one wave per
 // SIMD, which may use all 512.  Against the vector-ALU kernel, which read K
 // and V once per four rows: f16 D = 64, 777 tokens over 2,777 (14 / 2 heads),
-// 436 -> 33 us; bf16 D = 256, 512 over 4,700 soft-capped under a window mask
-// (16 / 8 heads), 3,033 -> 203 us.
+// 436 -> 29 us; bf16 D = 256, 512 over 4,700 soft-capped under a window mask
+// (16 / 8 heads), 3,033 -> 108 us.
 template <typename T, class Src, int FEAT, int NW, int D>
 __global__ __launch_bounds__(NW * 64, D == 256 ? 1 : 2) void chunk32_mfma_dim_kernel(AttnParams p,
                                                                                      Src src) {

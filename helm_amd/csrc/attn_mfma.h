@@ -31,8 +31,9 @@
 // (Written for D = 128; D = 64 halves the K chunks and the dims a lane holds
 // of a V row to four, D = 256 doubles both, the V row's halves apart: VRow.
 // Against the vector-ALU kernel that served them before: f16 D = 64, four
-// sequences of 3k-16k tokens, 45.6 -> 17.6 us; bf16 D = 256, 8,000 tokens
-// soft-capped under a window mask, 37.9 -> 19.2 us.)
+// sequences of 3k-16k tokens, 45.6 -> 17.4 us; bf16 D = 256, 8,000 tokens
+// soft-capped under a window mask, 37.9 -> 18.7 us.  Their weights' parts and
+// scale: weight_parts, weight_shift.)
 // No data moves between lanes in the loop; the split's per-wave states meet in
 // LDS; the shared split epilogue (attn_kernel.h) merges the waves and then
 // the splits.
@@ -231,7 +232,7 @@ __device__ __forceinline__ mf_u32x4 load16_any(const char* p) {
 // holds while their powers stay in fp32's range: |k| in [2^-20, 2^8], far around
 // every head dim and cap in use.  Any other step takes tanhf (for every step it
 // had cost as much as the softmax: bf16 chunk of 512 over 8,192, 32 / 8 heads,
-// 4,096-token window, capped: 236 us, now 134).
+// 4,096-token window, capped: 236 us, now 135).
 template <int N>
 __device__ __forceinline__ void softcap_scores(float (&x)[N], float k, float cap) {
   float top = fabsf(x[0]);
@@ -919,7 +920,7 @@ __device__ __forceinline__ void decode_mfma_body(const AttnParams& p, const Src&
     // the claim still in flight (its result is not needed)
     __builtin_amdgcn_s_waitcnt(0);
   } else
-  // ---- main loop: a ring of kMfmaBufs register buffers, kMfmaBufs - 1
+  // ---- main loop: a ring of mfma_bufs(D) register buffers, all but one
   // blocks' loads in flight while one block is computed ----------------------
   {
     constexpr int NB = mfma_bufs(D);

@@ -303,7 +303,8 @@ int balanced_pps(double pages, double units, int target, int lo_pps, int max_pps
 // mean share of the pages a query block walks (a causal first prompt: about
 // half).  Measured per 64-token stage (one workgroup alone / per workgroup on
 // a full CU, us): D = 128 four waves 2.0 / 1.6, eight waves 2.3; D = 64
-// 1.6 / 1.0; D = 256 3.3.  A split length from the number of workgroups alone gave
+// 1.6 / 1.0; D = 256 3.3 (f16; bf16's third weight part adds a sixth, about alike
+// for every split count).  A split length from the number of workgroups alone gave
 // 480-workgroup prompts a second split of a few pages and its partials (f16
 // 40 heads, 1,500 tokens: 97 us, one split 47; bf16 8 heads, 4,000 tokens: 85,
 // now 71).  The merge walks a row's splits, 0.04 us each.  Few KV heads over a long

@@ -1,5 +1,5 @@
 """What the weights of the matrix-core kernels at head dims 64 and 256 keep of
-their 32 bits, and what infinities, NaN and -inf masks give there."""
+their 32 bits, and what infinities, NaN and -inf masks give at 64, 128 and 256."""
 import math
 
 import pytest
@@ -117,6 +117,22 @@ def test_infinite_values(D, dtype, S, sizes):
     V[..., :4] = 0
     ref = A.attention_fp64_batched(q[0], K[0], V[0])
     assert (out[..., 4:] - ref[..., 4:]).abs().max().item() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("S", [1, 40])
+def test_infinite_values_at_head_dim_128_stay_in_their_column(dtype, S):
+    """D = 128, whose weights were parts from the start: the column of an
+    infinity is infinite or NaN, the others keep their values."""
+    D, T = 128, 200
+    q, K, V = _chunk(D, dtype, T, S, S)
+    V[:, :, 5, 0] = math.inf
+    out = perform_streaming_attention(q.to(DEV), _pages(K, V, [64, 64, 64, 8]),
+                                      attention_mask=_zero_mask(S, T))[0].double().cpu()
+    assert not out[..., 0].isfinite().any()
+    V[..., 0] = 0
+    ref = A.attention_fp64_batched(q[0], K[0], V[0])
+    assert (out[..., 1:] - ref[..., 1:]).abs().max().item() <= TOL[dtype]
 
 
 def _chunk(D, dtype, T, S, seed):
