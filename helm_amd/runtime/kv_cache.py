@@ -1298,7 +1298,7 @@ def _decode_contiguous_fast(kvcms, q: torch.Tensor, k: torch.Tensor, v: torch.Te
     (helm_decode_step): the attention kernel writes each item's token into its
     buffer's last virtual page itself, which saves the append launch, and the
     arguments go into this thread's block (four sequences of 8,200 tokens, 40 /
-    8 heads under a bf16 mask: 39.6 -> 27.1 us per step of one layer).  Every
+    8 heads under a bf16 mask: 40 -> 27.3-28.8 us per step of one layer).  Every
     item a KVCacheManager with room for the token, no write of its own queued,
     and buffers of the query's dtype and device.  Returns None, with nothing
     changed, when any of that does not hold."""

@@ -5,6 +5,7 @@ import math
 import pytest
 import torch
 
+from helm_amd.paged import paged_decode_attention
 from helm_amd.runtime.kv_cache import KVPage, perform_streaming_attention
 from oracle import attention as A
 
@@ -117,6 +118,46 @@ def test_infinite_values(D, dtype, S, sizes):
     V[..., :4] = 0
     ref = A.attention_fp64_batched(q[0], K[0], V[0])
     assert (out[..., 4:] - ref[..., 4:]).abs().max().item() <= TOL[dtype]
+
+
+@pytest.mark.parametrize("D", [64, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("route,cap", [
+    ("causal", None),                 # (a soft-capped prompt is not causal)
+    ("pool_decode", None), ("pool_decode", 20.0), ("pool_chunk", None), ("pool_chunk", 20.0)])
+def test_infinite_values_without_a_mask(D, dtype, route, cap):
+    """The same under the causal limit (the rows that see every infinity) and
+    over a slot pool, soft-capped or not, in one split and in several."""
+    T = 150 if route == "causal" else 700
+    S = {"causal": T, "pool_decode": 1, "pool_chunk": 40}[route]
+    g = torch.Generator().manual_seed(D + T)
+    K, V = (torch.randn(1, 2, T, D, generator=g).to(dtype) for _ in range(2))
+    q = torch.randn(1, 6, S, D, generator=g).to(dtype)
+    V[:, :, 5, 0] = math.inf
+    V[:, :, 7, 1] = -math.inf
+    V[:, :, 3, 2], V[:, :, 8, 2] = math.inf, -math.inf
+    if route == "causal":
+        outs = [perform_streaming_attention(q.to(DEV), _pages(K, V, [64, 64, 22]), softcap=cap)]
+    else:
+        pad = torch.zeros(1, 2, 704 - T, D, dtype=dtype)
+        pool = [torch.cat([x, pad], 2).reshape(2, 44, 16, D).transpose(0, 1).contiguous().to(DEV)
+                for x in (K, V)]
+        table = torch.arange(44, dtype=torch.int32, device=DEV)[None]
+        lens = torch.tensor([T], dtype=torch.int32, device=DEV)
+        outs = [paged_decode_attention(q.to(DEV), *pool, table, lens, softcap=cap,
+                                       pages_per_split=pps) for pps in (0, 44, 9)]
+    V[..., :3] = 0
+    mask = None
+    if route == "causal":
+        mask = torch.zeros(1, S, T).masked_fill_(
+            torch.arange(T)[None, :] > torch.arange(S)[:, None], -math.inf)
+    ref = A.attention_fp64_batched(q[0], K[0], V[0], mask=mask, softcap=cap)
+    seen = slice(8, None) if route == "causal" else slice(None)
+    for out in outs:
+        out = out[0].double().cpu()[:, seen]
+        assert (out[..., 0] == math.inf).all() and (out[..., 1] == -math.inf).all()
+        assert out[..., 2].isnan().all()
+        assert (out[..., 3:] - ref[:, seen, 3:]).abs().max().item() <= TOL[dtype]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
